@@ -1,7 +1,10 @@
 // Batched complex GEMM on the gfx950 matrix cores.
 //
-// Workgroup = 4 wave64s computing a 64 x 64 complex tile of C; each wave owns
-// a 32 x 32 quadrant = 2 x 2 blocks of the 16 x 16 MFMA output, kept as
+// The dispatch of every compute mode, and the FP32 and split-bf16 kernels (FP64
+// has its own file).
+//
+// FP32 workgroup = 4 wave64s computing a 64 x 64 complex tile of C; each wave
+// owns a 32 x 32 quadrant = 2 x 2 blocks of the 16 x 16 MFMA output, kept as
 // separate real / imaginary accumulators (4 real MFMAs per complex block and
 // k-step: re += ar*br - ai*bi, im += ar*bi + ai*br).
 //
@@ -19,12 +22,11 @@
 // once and walks several batches.  Each call site is its own kernel symbol;
 // the launch variant per site comes from the built-in choice, a per-thread
 // table (the plan's autotuned choice) or a global override.
-#include "zgemm.hpp"
+#include "tiling.hpp"
 #include "ozaki.hpp"
 
 #include <algorithm>
 #include <cstdio>
-#include <type_traits>
 
 namespace ggpu {
 namespace {
@@ -35,89 +37,23 @@ constexpr int BKT = 16;
 constexpr int NTHREADS = 256;
 constexpr int PAD = 2;
 
-typedef double v4d __attribute__((ext_vector_type(4)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <class T> struct Cplx;
-template <> struct Cplx<double> { using type = double2; };
-template <> struct Cplx<float> { using type = float2; };
-
-template <class T, class V>
-__device__ inline V mfma(T a, T b, V c);
-template <>
-__device__ inline v4d mfma<double, v4d>(double a, double b, v4d c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-template <>
-__device__ inline v4f mfma<float, v4f>(float a, float b, v4f c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <class T> struct Acc;
-template <> struct Acc<double> { using type = v4d; };
-template <> struct Acc<float> { using type = v4f; };
-
 // Row (within the 16 x 16 block) of accumulator register r of lane group
-// lk = lane / 16.  Measured on gfx950: v_mfma_f64_16x16x4_f64 holds rows
-// lk + 4 r, v_mfma_f32_16x16x4_f32 holds rows 4 lk + r; the column is lane % 16
-// for both.
-template <class T> __device__ inline int acc_row(int lk, int r);
-template <> __device__ inline int acc_row<double>(int lk, int r) { return lk + 4 * r; }
-template <> __device__ inline int acc_row<float>(int lk, int r) { return 4 * lk + r; }
-
-// Workgroup -> tile mapping.  Workgroups are dispatched round-robin over the
-// 8 XCDs (each with its own L2); the linear id is remapped so that every XCD
-// receives a contiguous range of logical tiles, ordered m-tile fastest, then
-// n-tile, then batch: the workgroups that share a B panel (same n-tile) and an
-// A panel (same batch) run on the same XCD at the same time.
-constexpr int NXCD = 8;
-__device__ inline int64_t xcd_logical(int64_t id, int64_t total) {
-  const int64_t xcd = id % NXCD, slot = id / NXCD;
-  const int64_t per = total / NXCD, rem = total % NXCD;
-  return (xcd < rem) ? xcd * (per + 1) + slot : rem * (per + 1) + (xcd - rem) * per + slot;
-}
-
-// Logical tile -> (m-tile, n-tile, batch b0, batch b1).  Default order:
-// m-tile fastest, then n-tile, then batch.  With d.batch_major the batch
-// index runs fastest instead: chosen when every batch shares A (A's batch
-// strides are zero), so the workgroups reusing one A panel run back to back
-// and find it in L2 instead of re-reading A from memory once per batch.
-struct TileCoord { int mt, nt; int64_t b0, b1; };
-__device__ inline TileCoord tile_coord(const GemmDesc& d, int tiles_m, int tiles_n) {
-  int64_t lg = xcd_logical(blockIdx.x, gridDim.x);
-  TileCoord c;
-  if (d.batch_major) {
-    const int64_t nb = (int64_t)d.nb0 * d.nb1;
-    const int64_t b = lg % nb;
-    lg /= nb;
-    c.mt = (int)(lg % tiles_m);
-    c.nt = (int)(lg / tiles_m);
-    c.b1 = b % d.nb1;
-    c.b0 = b / d.nb1;
-  } else {
-    c.mt = (int)(lg % tiles_m);
-    lg /= tiles_m;
-    c.nt = (int)(lg % tiles_n);
-    lg /= tiles_n;
-    c.b1 = lg % d.nb1;
-    c.b0 = lg / d.nb1;
-  }
-  return c;
-}
-
-// T: arithmetic type of operands and MFMA; TO: complex element type of C.
+// lk = lane / 16 is 4 lk + r, the column lane % 16 (measured on gfx950).
+// FP32 kernel.  TO: complex element type of C.
 // AKC: A's k index is the contiguous one (else its m index).
 // BKC: B's k index is the contiguous one (else its n index).
-// GAUSS: 3 real products per complex product (t1 = ar br, t2 = ai bi,
-//   t3 = (ar + ai)(br + bi); re = t1 - t2, im = t3 - t1 - t2) instead of 4.
+// 4 real products per complex product.
 // BK: k per LDS stage (16, or 8 for half the LDS and twice the workgroups
 // per CU).
 // WPE: waves per SIMD the register allocation must allow (1: no constraint).
-template <class T, class TO, bool AKC, bool BKC, bool GAUSS, int SITE, int BK = BKT, int WPE = 1>
+template <class TO, bool AKC, bool BKC, int SITE, int BK = BKT, int WPE = 1>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_mfma_kernel(
     const GemmDesc d) {
-  using CT = typename Cplx<T>::type;
-  using AV = typename Acc<T>::type;
+  using T = float;
+  using CT = c32;
+  using AV = v4f;
   constexpr int EPT = BM * BK / NTHREADS;   // complex elements per thread and operand
   __shared__ T sA[2][2][BK][BM + PAD];   // [buffer][re/im][k][m]
   __shared__ T sB[2][2][BK][BN + PAD];   // [buffer][re/im][k][n]
@@ -175,9 +111,9 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
   const int lane = tid & 63, w = tid >> 6;
   const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
   const int lr = lane & 15, lk = lane >> 4;
-  AV acc[GAUSS ? 3 : 2][2][2];
+  AV acc[2][2][2];
 #pragma unroll
-  for (int a = 0; a < (GAUSS ? 3 : 2); ++a)
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -193,32 +129,18 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
       br[i] = sB[buf][0][kk + lk][wn + 16 * i + lr];
       bi[i] = sB[buf][1][kk + lk][wn + 16 * i + lr];
     }
-    if (GAUSS) {
-      T as[2], bs[2];
+    T nai[2];
 #pragma unroll
-      for (int i = 0; i < 2; ++i) { as[i] = ar[i] + ai[i]; bs[i] = br[i] + bi[i]; }
+    for (int i = 0; i < 2; ++i) nai[i] = -ai[i];
 #pragma unroll
-      for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          acc[0][i][j] = mfma<T, AV>(ar[i], br[j], acc[0][i][j]);
-          acc[1][i][j] = mfma<T, AV>(ai[i], bi[j], acc[1][i][j]);
-          acc[GAUSS ? 2 : 0][i][j] = mfma<T, AV>(as[i], bs[j], acc[GAUSS ? 2 : 0][i][j]);
-        }
-    } else {
-      T nai[2];
-#pragma unroll
-      for (int i = 0; i < 2; ++i) nai[i] = -ai[i];
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          acc[0][i][j] = mfma<T, AV>(ar[i], br[j], acc[0][i][j]);
-          acc[1][i][j] = mfma<T, AV>(ar[i], bi[j], acc[1][i][j]);
-          acc[0][i][j] = mfma<T, AV>(nai[i], bi[j], acc[0][i][j]);
-          acc[1][i][j] = mfma<T, AV>(ai[i], br[j], acc[1][i][j]);
-        }
-    }
+      for (int j = 0; j < 2; ++j) {
+        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[i], br[j], acc[0][i][j], 0, 0, 0);
+        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[i], bi[j], acc[1][i][j], 0, 0, 0);
+        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(nai[i], bi[j], acc[0][i][j], 0, 0, 0);
+        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai[i], br[j], acc[1][i][j], 0, 0, 0);
+      }
   };
 
   // All k-steps of k-tile it (LDS buffer it & 1).
@@ -249,18 +171,10 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + 16 * i + acc_row<T>(lk, r);
+        const int row = m0 + wm + 16 * i + 4 * lk + r;
         const int col = n0 + wn + 16 * j + lr;
         if (row < d.M && col < d.N) {
-          double xr, xi;
-          if (GAUSS) {
-            const double t1 = acc[0][i][j][r], t2 = acc[1][i][j][r], t3 = acc[GAUSS ? 2 : 0][i][j][r];
-            xr = t1 - t2;
-            xi = t3 - t1 - t2;
-          } else {
-            xr = acc[0][i][j][r];
-            xi = acc[1][i][j][r];
-          }
+          const double xr = acc[0][i][j][r], xi = acc[1][i][j][r];
           double vr = d.alpha_re * xr - d.alpha_im * xi;
           double vi = d.alpha_re * xi + d.alpha_im * xr;
           TO* p = C + row * d.C.rs + col * d.C.cs;
@@ -1217,56 +1131,49 @@ void launch_bf16x3(const GemmDesc& d, hipStream_t stream, int v) {
   }
 }
 
-template <class T, class TO, bool GAUSS, int SITE, int BK, int WPE>
-void launch_site_bk(const GemmDesc& d, hipStream_t stream) {
+template <class TO, int SITE, int BK, int WPE>
+void launch_f32_bk(const GemmDesc& d, hipStream_t stream) {
   const int64_t tiles = (int64_t)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN);
   const int64_t total = tiles * d.nb0 * d.nb1;
   require(total < (int64_t)1 << 31, "gemm: grid too large");
   dim3 grid((unsigned)total), block(NTHREADS);
   const bool akc = (d.A.cs == 1) || (d.A.rs != 1);
   const bool bkc = (d.B.rs == 1) || (d.B.cs != 1);
-  if (akc && bkc) hipLaunchKernelGGL((gemm_mfma_kernel<T, TO, true, true, GAUSS, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else if (akc) hipLaunchKernelGGL((gemm_mfma_kernel<T, TO, true, false, GAUSS, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else if (bkc) hipLaunchKernelGGL((gemm_mfma_kernel<T, TO, false, true, GAUSS, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else hipLaunchKernelGGL((gemm_mfma_kernel<T, TO, false, false, GAUSS, SITE, BK, WPE>), grid, block, 0, stream, d);
+  if (akc && bkc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, true, true, SITE, BK, WPE>), grid, block, 0, stream, d);
+  else if (akc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, true, false, SITE, BK, WPE>), grid, block, 0, stream, d);
+  else if (bkc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, false, true, SITE, BK, WPE>), grid, block, 0, stream, d);
+  else hipLaunchKernelGGL((gemm_mfma_kernel<TO, false, false, SITE, BK, WPE>), grid, block, 0, stream, d);
   GGPU_HIP(hipGetLastError());
 }
 
-template <class T, class TO, bool GAUSS, int SITE>
-void launch_site(const GemmDesc& d, hipStream_t stream, int variant) {
+template <class TO, int SITE>
+void launch_f32_site(const GemmDesc& d, hipStream_t stream, int variant) {
   // Variants measured on MI355X (nao = 52, NQ = 300, nts = 110; medians of
   // interleaved rounds): staging 8 k per LDS step is faster than 16 or equal
-  // at every call site, and FP64 register allocation for three waves per
-  // SIMD (152-156 VGPRs, accumulators out of the AGPRs, no spills) instead
-  // of two gains 7-17 % at every site.  FP32 runs five waves unconstrained.
-  // All variants give the same sums bit for bit.
-  constexpr bool f64 = std::is_same<T, double>::value;
-  constexpr int pref = f64 ? 83 : 8;
-  switch (variant > 0 ? variant : pref) {
-    case 8: return launch_site_bk<T, TO, GAUSS, SITE, 8, 1>(d, stream);
-    case 83: return launch_site_bk<T, TO, GAUSS, SITE, 8, 3>(d, stream);
-    case 84: return launch_site_bk<T, TO, GAUSS, SITE, 8, 4>(d, stream);
-    default: return launch_site_bk<T, TO, GAUSS, SITE, 16, 1>(d, stream);
+  // at every call site; FP32 runs five waves unconstrained.  All variants give
+  // the same sums bit for bit.
+  switch (variant > 0 ? variant : 8) {
+    case 8: return launch_f32_bk<TO, SITE, 8, 1>(d, stream);
+    case 83: return launch_f32_bk<TO, SITE, 8, 3>(d, stream);
+    default: return launch_f32_bk<TO, SITE, 16, 1>(d, stream);
   }
 }
 
-// FP64 uses the 3-product (Gauss) complex scheme; FP32 keeps 4 products
-// (the Gauss recombination t3 - t1 - t2 loses relative accuracy when the
-// result is small against |A||B|, which FP32 cannot afford).
-template <class T, class TO>
-void launch_typed(const GemmDesc& d, hipStream_t stream, int v) {
-  constexpr bool G = std::is_same<T, double>::value;
+// FP32 keeps 4 products per complex product (the Gauss recombination
+// t3 - t1 - t2 of the FP64 kernel loses relative accuracy when the result is
+// small against |A||B|, which FP32 cannot afford).
+template <class TO>
+void launch_f32(const GemmDesc& d, hipStream_t stream, int v) {
   switch (d.site) {
-    case kSiteP0X1: launch_site<T, TO, G, kSiteP0X1>(d, stream, v); break;
-    case kSiteP0X2: launch_site<T, TO, G, kSiteP0X2>(d, stream, v); break;
-    case kSiteP0: launch_site<T, TO, G, kSiteP0>(d, stream, v); break;
-    case kSiteSigY1: launch_site<T, TO, G, kSiteSigY1>(d, stream, v); break;
-    case kSiteSigY2: launch_site<T, TO, G, kSiteSigY2>(d, stream, v); break;
-    case kSiteSigma: launch_site<T, TO, G, kSiteSigma>(d, stream, v); break;
-    default: launch_site<T, TO, G, kSiteOther>(d, stream, v); break;
+    case kSiteP0X1: launch_f32_site<TO, kSiteP0X1>(d, stream, v); break;
+    case kSiteP0X2: launch_f32_site<TO, kSiteP0X2>(d, stream, v); break;
+    case kSiteP0: launch_f32_site<TO, kSiteP0>(d, stream, v); break;
+    case kSiteSigY1: launch_f32_site<TO, kSiteSigY1>(d, stream, v); break;
+    case kSiteSigY2: launch_f32_site<TO, kSiteSigY2>(d, stream, v); break;
+    case kSiteSigma: launch_f32_site<TO, kSiteSigma>(d, stream, v); break;
+    default: launch_f32_site<TO, kSiteOther>(d, stream, v); break;
   }
 }
-
 
 // Range of element offsets (relative to ptr) touched by a 2-D view with the
 // given extents and strides, over all batch indices.
@@ -1366,11 +1273,11 @@ void gemm(const GemmDesc& dd, hipStream_t stream) {
   switch (d.compute) {
     case Compute::F64:
       require(!d.out_f32, "gemm: FP64 compute writes complex128");
-      launch_typed<double, double2>(d, stream, v);
+      launch_f64(d, stream, v);
       break;
     case Compute::F32:
-      if (d.out_f32) launch_typed<float, float2>(d, stream, v);
-      else launch_typed<float, double2>(d, stream, v);
+      if (d.out_f32) launch_f32<float2>(d, stream, v);
+      else launch_f32<double2>(d, stream, v);
       break;
     case Compute::BF16X3:
       if (d.out_f32) launch_bf16x3<float2>(d, stream, v);
@@ -1387,7 +1294,7 @@ void gemm(const GemmDesc& dd, hipStream_t stream) {
         require(!d.out_f32, "gemm: FP64 kernel writes complex128");
         GemmDesc f = d;
         f.compute = Compute::F64;
-        launch_typed<double, double2>(f, stream, v);
+        launch_f64(f, stream, v);
       }
       break;
     }

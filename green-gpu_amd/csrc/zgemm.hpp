@@ -103,16 +103,17 @@ enum {
 // Variant of a Compute::I8X5 / I8X4 launch that runs the int8 emulation with
 // the mode's slice count; kVariantInt8x5 runs it with five slices in either
 // mode (FP64-accurate products, so any site of a four-slice plan may take
-// it); the FP64 kernel variants (8, 16, 83, 84) run the launch on the FP64
+// it); the FP64 kernel variants (8, 16, 83) run the launch on the FP64
 // kernel instead.  Built-in choice: the emulation at the Sigma P.Y1 product
 // and the P0 contraction (the sites where it is faster on the benchmark
 // shapes), the FP64 kernel everywhere else; per-site variants override it.
 enum { kVariantInt8 = 200, kVariantInt8x5 = 201 };
 // Launch variant per call site for the launches of the calling thread
 // (table of kNumSites entries, -1: the built-in choice; nullptr: none):
-// for FP64 / FP32 8 or 16 forces the LDS k-depth, 83 or 84 k-depth 8 with
-// registers allocated for 3 or 4 waves per SIMD (all give the same sums);
-// for split-bf16 a kBf16Tile* value; in the int8 modes kVariantInt8 or an
+// for FP64 8 or 16 forces the 64 x 64 or 48 x 64 workgroup tile and 83 takes
+// the tile chosen by the shape; for FP32 8 or 16 forces the LDS k-depth, 83
+// k-depth 8 with registers allocated for 3 waves per SIMD (all give the same
+// sums); for split-bf16 a kBf16Tile* value; in the int8 modes kVariantInt8 or an
 // FP64 kernel variant.
 void set_site_variants(const int* table);
 // Device workspace of the Compute::I8X5 / I8X4 launches of the calling thread
@@ -149,6 +150,11 @@ struct GemmDesc {
 // Throws Error(kErrArgument) if any address the launch would touch falls
 // outside an operand's declared allocation.
 void gemm_check_bounds(const GemmDesc& d);
+
+// The FP64 kernel of a checked descriptor with M, N > 0 (gemm() calls it);
+// variant 8: the 64 x 64 tile, 16: the 48 x 64 tile, others: the tile its rule
+// picks for the shape.
+void launch_f64(const GemmDesc& d, hipStream_t stream, int variant);
 
 // Enqueue the GEMM on `stream`.
 void gemm(const GemmDesc& d, hipStream_t stream);
