@@ -225,28 +225,30 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WP
 
 // The menu of workgroup tiles: rows, columns, waves per SIMD that the
 // registers (24 accumulator registers per 16 x 16 block and wave) and LDS
-// leave.  All give the same sums.
+// leave, and the tile's own time per area against the others'.  All give the
+// same sums.
 enum Tile { k64x64, k48x64, k64x32, k64x48, k64x80, k64x96, k64x112, k80x64, k32x64, k64x16, k32x32, kTiles };
-struct TileShape { int m, n, waves; };
-constexpr TileShape kTileShape[kTiles] = {{64, 64, 3}, {48, 64, 4}, {64, 32, 5},  {64, 48, 4}, {64, 80, 3}, {64, 96, 2},
-                                          {64, 112, 2}, {80, 64, 3}, {32, 64, 5}, {64, 16, 6}, {32, 32, 6}};
+struct TileShape { int m, n, waves; double time; };
+constexpr TileShape kTileShape[kTiles] = {
+    {64, 64, 3, 0.95}, {48, 64, 4, 1.0},  {64, 32, 5, 0.95}, {64, 48, 4, 1.05}, {64, 80, 3, 1.0}, {64, 96, 2, 1.0},
+    {64, 112, 2, 1.0}, {80, 64, 3, 1.0}, {32, 64, 5, 0.95}, {64, 16, 6, 1.1},  {32, 32, 6, 1.0}};
 
 // Expected time of a launch in units of matrix-pipe work per CU: the padded
 // tile area each of the 256 CUs gets through (whole rounds while the grid
 // fills the chip only a few times), slower by 1 + 0.3 / n with n waves per
 // SIMD to hide latencies, plus the tile's operand traffic (rows + columns).
-// Fitted to 42 shapes of the HF / GW contractions (nao 16 to 104, NQ 64 to
+// Fitted to 60 shapes of the HF / GW contractions (nao 10 to 104, NQ 64 to
 // 600) timed with every tile: the choice is within 1 % of the fastest tile on
-// (geometric) average.  Against the 64 x 64 tile that every launch had before
-// it is 1.3 - 2.2x faster where an extent is just above a multiple of 64
-// (nao = 72: p0_gvh 45 -> 69 TFLOP/s) or the grid is small (nao = 26,
-// NQ = 100: p0_contract 15 -> 30, sig_vg 18 -> 34, sig_py 43 -> 54).
+// (geometric) average.  Against a 64 x 64 tile everywhere it is 1.3 - 2.2x
+// faster where an extent is just above a multiple of 64 (nao = 72: p0_gvh
+// 46 -> 69 TFLOP/s) or the grid is small (nao = 26, NQ = 100: p0_contract
+// 20 -> 33, sig_vg 20 -> 36).
 double tile_cost(const GemmDesc& d, const TileShape& t) {
   const double tiles = (double)((d.M + t.m - 1) / t.m) * ((d.N + t.n - 1) / t.n) * d.nb0 * d.nb1;
   double rounds = tiles / 256.0;
-  if (rounds <= 4.0 * t.waves) rounds = std::ceil(rounds);
+  if (rounds <= 8.0 * t.waves) rounds = std::ceil(rounds);
   const double n = std::min<double>(t.waves, std::max(1.0, std::ceil(tiles / 256.0)));
-  return rounds * ((double)t.m * t.n * (1.0 + 0.3 / n) + 2.0 * (t.m + t.n));
+  return t.time * rounds * ((double)t.m * t.n * (1.0 + 0.3 / n) + 3.0 * (t.m + t.n));
 }
 
 Tile choose_tile(const GemmDesc& d) {
@@ -274,7 +276,7 @@ template <bool AKC, bool BKC, int SITE>
 void launch_tile(const GemmDesc& d, hipStream_t stream, Tile t) {
   switch (t) {
     case k48x64: return launch_one<1, 4, 3, 1, 4, AKC, BKC, SITE>(d, stream);
-    case k64x32: return launch_one<4, 1, 1, 2, 5, AKC, BKC, SITE>(d, stream);
+    case k64x32: return launch_one<2, 2, 2, 1, 5, AKC, BKC, SITE>(d, stream);
     case k64x48: return launch_one<4, 1, 1, 3, 4, AKC, BKC, SITE>(d, stream);
     case k64x80: return launch_one<4, 1, 1, 5, 3, AKC, BKC, SITE>(d, stream);
     case k64x96: return launch_one<4, 1, 1, 6, 2, AKC, BKC, SITE>(d, stream);
