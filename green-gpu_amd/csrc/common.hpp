@@ -78,4 +78,24 @@ class DeviceBuffer {
   size_t n_ = 0;
 };
 
+// Owning pinned host allocation (device kernels may write it directly).
+template <class T>
+class PinnedBuffer {
+ public:
+  PinnedBuffer() = default;
+  ~PinnedBuffer() {
+    if (p_) (void)hipHostFree(p_);
+  }
+  PinnedBuffer(const PinnedBuffer&) = delete;
+  PinnedBuffer& operator=(const PinnedBuffer&) = delete;
+  void allocate(size_t n) {
+    require(p_ == nullptr, "pinned buffer: already allocated", kErrState);
+    GGPU_HIP(hipHostMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T), hipHostMallocDefault));
+  }
+  T* get() const { return p_; }
+
+ private:
+  T* p_ = nullptr;
+};
+
 }  // namespace ggpu

@@ -10,6 +10,7 @@
 //   work      pair-batch intermediates (X1, X2 for P0; Y1, Y2 for Sigma)
 #include "engine.hpp"
 #include "ozaki.hpp"
+#include "hf.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -413,6 +414,18 @@ void unfold_pairs(IntegralStore& st, const PairTable& tab, int i0, int n, const 
   c.conj = tab.conj.get() + i0;
   block_copy(c, s);
   st.done(s);
+}
+
+// The blocks of pairs [i0, i0 + n) of a table where the store holds them (or
+// stages them: call store.done() after the last read), checked on the host.
+static PairBlocks pair_blocks(IntegralStore& st, const PairTable& tab, int i0, int n, int64_t stride, hipStream_t s) {
+  for (int i = i0; i < i0 + n; ++i)
+    require((tab.host[i].pos + 1) * stride <= st.elems(), "pair_blocks: pair outside store");
+  PairBlocks v;
+  v.base = st.view(tab, i0, n, s, &v.off);
+  v.trans = tab.trans.get() + i0;
+  v.conj = tab.conj.get() + i0;
+  return v;
 }
 
 // ---------------------------------------------------------------------------
@@ -1534,6 +1547,9 @@ HfPlan::HfPlan(int nao_, int nso_, int ns_, int NQ_, const ggpu_symmetry& s)
   Kpart.resize((size_t)nsplit * nps * n2);
   Kout.resize((size_t)sym.ink * nps * n2);
   jvec.resize(NQ);
+  jpart.resize((size_t)sym.nk * NQ);
+  F_dev.resize((size_t)ns * sym.ink * so2);
+  traces.allocate((size_t)ns * sym.ink);
   S_dev.resize((size_t)ns * sym.ink * so2);
   Ftmp.resize((size_t)nps * sym.ink * n2);
   diag_tables.resize(2);
@@ -1566,7 +1582,6 @@ HfPlan::HfPlan(int nao_, int nso_, int ns_, int NQ_, const ggpu_symmetry& s)
   }
   if (x2c) {
     dm2c_fbz.resize((size_t)sym.nk * so2);
-    F2c.resize((size_t)sym.ink * so2);
     build_split(x2c_split, sym.nk, 3, nao, so2, n2);
     // Fock blocks aa, bb, ab from Kout[ik][0..2]; ba = ab^dagger
     // (copy_2c_Fock_from_device_to_host, cuda_common.cu:176-205)
@@ -1670,15 +1685,8 @@ void HfPlan::exchange_device(z64* kpart, int nsp) {
         gemm_on(f, wk, wk, Span{kpart, (size_t)part_elems}, stream, kSiteHF);
       }
     }
-    sum_partials(kpart, (int64_t)nps * n2, nsp, Kout.get() + (int64_t)ik * nps * n2, (int64_t)nps * n2, stream);
+    sum_slices(kpart, 0, (int64_t)nps * n2, nsp, Kout.get() + (int64_t)ik * nps * n2, 0, (int64_t)nps * n2, 1, stream);
   }
-}
-
-static void ibz_to_host_layout(const std::vector<z64>& h, double* out, int ink, int ns, int64_t n2) {
-  z64* o = reinterpret_cast<z64*>(out);
-  for (int ik = 0; ik < ink; ++ik)
-    for (int s = 0; s < ns; ++s)
-      std::memcpy(o + ((int64_t)s * ink + ik) * n2, h.data() + ((int64_t)ik * ns + s) * n2, n2 * sizeof(z64));
 }
 
 void HfPlan::stage_dm(const z64* dm_dev) {
@@ -1691,19 +1699,25 @@ void HfPlan::stage_dm(const z64* dm_dev) {
   }
 }
 
-void HfPlan::fetch(double* out) {
-  const int64_t n2 = (int64_t)nao * nao;
-  (void)store.collect_staging_ms();   // staging timers are not reported for HF
-  if (x2c) {
-    spinor_copy(x2c_merge, Kout.get(), Kout.size(), nao, 0, F2c.get(), F2c.size(), nso, 0, nao, 1, 1.0, stream);
-    GGPU_HIP(hipMemcpyAsync(out, F2c.get(), F2c.bytes(), hipMemcpyDeviceToHost, stream));
-    GGPU_HIP(hipStreamSynchronize(stream));
-    return;
+// Kout in the caller's layout on the device.
+void HfPlan::to_caller_layout(z64* out) {
+  const int64_t n2 = (int64_t)nao * nao, so2 = (int64_t)nso * nso;
+  if (x2c)
+    spinor_copy(x2c_merge, Kout.get(), Kout.size(), nao, 0, out, (size_t)sym.ink * so2, nso, 0, nao, 1, 1.0, stream);
+  else
+    slab_gather(Kout.get(), kout_src.get(), out, kout_dst.get(), (int)kout_src.size(), n2, 1.0, stream);
+}
+
+void HfPlan::fetch(double* out, bool with_energy) {
+  to_caller_layout(F_dev.get());
+  if (with_energy) {
+    energy_valid = false;
+    enqueue_traces();   // read back with the Fock matrices: one wait
   }
-  std::vector<z64> h(Kout.size());
-  GGPU_HIP(hipMemcpyAsync(h.data(), Kout.get(), Kout.bytes(), hipMemcpyDeviceToHost, stream));
+  GGPU_HIP(hipMemcpyAsync(out, F_dev.get(), F_dev.bytes(), hipMemcpyDeviceToHost, stream));
   GGPU_HIP(hipStreamSynchronize(stream));
-  ibz_to_host_layout(h, out, sym.ink, ns, n2);
+  (void)store.collect_staging_ms();   // staging timers are not reported for HF
+  if (with_energy) collect_energy();
 }
 
 // E_2 = (1/nk) sum_{s, k in IBZ} w_k (1/2) Re Tr[D_s(k) F_s(k)], w_k = |star(k)|:
@@ -1712,27 +1726,17 @@ void HfPlan::fetch(double* out) {
 // reference returns only the Fock matrix (hf_gpu_kernel.cpp:66-104); the
 // energy is green-mbpt's.  With ns = 1 the density is the spin-summed one, so
 // the same formula holds.  Traces accumulate in FP64 on the device.
-void HfPlan::compute_energy() {
+void HfPlan::enqueue_traces() {
   const int n = x2c ? nso : nao;
   const int64_t n2 = (int64_t)n * n;
-  const int nsp = x2c ? 1 : ns;
-  traces.resize((size_t)nsp * sym.ink);
-  GemmDesc g;   // tr[s][ik] = sum_a sum_b D[a][b] F[b][a]: K index b, K-batch a
-  g.M = 1; g.N = 1; g.K = n; g.KB = n; g.nb0 = nsp; g.nb1 = sym.ink;
-  g.A.ptr = dm_host_dev.get(); g.A.rs = 0; g.A.cs = 1; g.A.kbs = n;
-  g.A.bs0 = (int64_t)sym.ink * n2; g.A.bs1 = n2;
-  const z64* F = x2c ? F2c.get() : Kout.get();
-  g.B.ptr = F; g.B.rs = n; g.B.cs = 0; g.B.kbs = 1;
-  g.B.bs0 = x2c ? 0 : n2; g.B.bs1 = x2c ? n2 : (int64_t)ns * n2;
-  g.C.ptr = traces.get(); g.C.rs = 0; g.C.cs = 0; g.C.bs0 = sym.ink; g.C.bs1 = 1;
-  if (x2c) gemm_on(g, dm_host_dev, F2c, traces, stream, kSiteHF);
-  else gemm_on(g, dm_host_dev, Kout, traces, stream, kSiteHF);
-  std::vector<z64> h(traces.size());
-  GGPU_HIP(hipMemcpyAsync(h.data(), traces.get(), traces.bytes(), hipMemcpyDeviceToHost, stream));
-  GGPU_HIP(hipStreamSynchronize(stream));
+  density_traces(dm_host_dev.get(), F_dev.get(), n2, (int64_t)sym.ink * n2, n, ns, sym.ink, traces.get(), stream);
+}
+
+void HfPlan::collect_energy() {
   double e = 0.0;
-  for (int s = 0; s < nsp; ++s)
-    for (int ik = 0; ik < sym.ink; ++ik) e += (double)sym.k_stars[ik].size() * 0.5 * h[(size_t)s * sym.ink + ik].x;
+  for (int s = 0; s < ns; ++s)
+    for (int ik = 0; ik < sym.ink; ++ik)
+      e += (double)sym.k_stars[ik].size() * 0.5 * traces.get()[(size_t)s * sym.ink + ik].x;
   energy = e / sym.nk;
   energy_valid = true;
 }
@@ -1743,7 +1747,7 @@ void HfPlan::exchange(const double* dm, double* K) {
   GGPU_HIP(hipMemcpyAsync(dm_host_dev.get(), dm, dm_host_dev.bytes(), hipMemcpyHostToDevice, stream));
   stage_dm(dm_host_dev.get());
   exchange_device(Kpart.get(), nsplit);
-  fetch(K);
+  fetch(K, false);
 }
 
 // The exchange on caller device buffers with the K partial sums in the static
@@ -1756,7 +1760,7 @@ void HfPlan::exchange_device_noalloc(const z64* dm_dev, z64* K_dev) {
   require(!store.staged(), "hf no-alloc exchange: needs the integrals resident in HBM", kErrState);
   require(!complex64_operands(compute) || dm32.size() == dm_fbz.size(),
           "hf: reduced-precision density buffer missing");
-  const int64_t n2 = (int64_t)nao * nao, so2 = (int64_t)nso * nso;
+  const int64_t n2 = (int64_t)nao * nao;
   const int64_t slice = (int64_t)nps * n2;
   require(slice <= scratch_elems,
           "hf no-alloc exchange: one partial slice of " + std::to_string(slice) +
@@ -1765,10 +1769,7 @@ void HfPlan::exchange_device_noalloc(const z64* dm_dev, z64* K_dev) {
   const int nsp = (int)std::max<int64_t>(1, std::min<int64_t>(nsplit, scratch_elems / slice));
   stage_dm(dm_dev);
   exchange_device(scratch, nsp);
-  if (x2c)
-    spinor_copy(x2c_merge, Kout.get(), Kout.size(), nao, 0, K_dev, (size_t)sym.ink * so2, nso, 0, nao, 1, 1.0, stream);
-  else
-    slab_gather(Kout.get(), kout_src.get(), K_dev, kout_dst.get(), (int)kout_src.size(), n2, 1.0, stream);
+  to_caller_layout(K_dev);
   GGPU_HIP(hipStreamSynchronize(stream));
 }
 
@@ -1785,36 +1786,25 @@ void HfPlan::solve(const double* dm, const double* S_k, double madelung, double*
   // Hartree: jvec[Q] = (1/nk) sum_{k', s} sum_{a,b} V^Q(k',k')[a][b] D_s(k')[b][a]
   // (X2C: the density is D_aa + D_bb, blocks 0 and 1)
   const int nj = x2c ? 2 : ns;
-  z64* Vdir = work.get();
-  zero(jvec.get(), jvec.size(), stream);
-  for (int i0 = 0; i0 < sym.nk; i0 += kb) {
-    const int n = std::min(kb, sym.nk - i0);
-    unfold_pairs(store, diag_tables[0], i0, n, bidx_off.get(), Vdir, 0, NQ, nao, stream);
-    for (int b = 0; b < n; ++b)
-      for (int s = 0; s < nj; ++s) {
-        GemmDesc g;   // (NQ x 1) = sum_a sum_b V[Q][a][b] D[b][a]: K index b, K-batch a
-        g.M = NQ; g.N = 1; g.K = nao; g.KB = nao;
-        g.A.ptr = Vdir + b * stride; g.A.rs = n2; g.A.cs = 1; g.A.kbs = nao;
-        g.B.ptr = dm_fbz.get() + ((int64_t)(i0 + b) * nps + s) * n2; g.B.rs = nao; g.B.cs = 0; g.B.kbs = 1;
-        g.C.ptr = jvec.get(); g.C.rs = 1; g.C.cs = 1;
-        g.alpha_re = 1.0 / sym.nk; g.beta_re = 1.0;
-        gemm_on(g, work, dm_fbz, jvec, stream, kSiteHF);
-      }
-  }
-  // F[ik][s] = K + sum_Q jvec[Q] V^Q(k,k) - c madelung S D S
-  for (int i0 = 0; i0 < sym.ink; i0 += kb) {
-    const int n = std::min(kb, sym.ink - i0);
-    unfold_pairs(store, diag_tables[1], i0, n, bidx_off.get(), Vdir, 0, NQ, nao, stream);
-    for (int b = 0; b < n; ++b) {
-      GemmDesc g;   // (1 x nao^2) += jvec^T (1 x NQ) . V (NQ x nao^2), for every spin (X2C: aa, bb)
-      g.M = 1; g.N = (int)n2; g.K = NQ; g.nb0 = nj;
-      g.A.ptr = jvec.get(); g.A.rs = 0; g.A.cs = 1;
-      g.B.ptr = Vdir + b * stride; g.B.rs = n2; g.B.cs = 1;
-      g.C.ptr = Kout.get() + (int64_t)(i0 + b) * nps * n2; g.C.rs = 0; g.C.cs = 1; g.C.bs0 = n2;
-      g.beta_re = 1.0;
-      gemm_on(g, jvec, work, Kout, stream, kSiteHF);
+  // the stored diagonal pairs are read where they lie: all at once when
+  // resident, in staged batches otherwise
+  auto diagonal = [&](const PairTable& tab, auto&& f) {
+    const int total = (int)tab.host.size(), step = store.staged() ? kb : total;
+    for (int i0 = 0; i0 < total; i0 += step) {
+      const int n = std::min(step, total - i0);
+      f(i0, n, pair_blocks(store, tab, i0, n, stride, stream));
+      store.done(stream);
     }
-  }
+  };
+  diagonal(diag_tables[0], [&](int i0, int n, const PairBlocks& v) {
+    hartree_vector(v, n, NQ, nao, dm_fbz.get() + (int64_t)i0 * nps * n2, nps, nj, 1.0 / sym.nk,
+                   jpart.get() + (int64_t)i0 * NQ, stream);
+  });
+  sum_slices(jpart.get(), 0, NQ, sym.nk, jvec.get(), 0, NQ, 1, stream);
+  // F[ik][s] = K + sum_Q jvec[Q] V^Q(k,k) - c madelung S D S
+  diagonal(diag_tables[1], [&](int i0, int n, const PairBlocks& v) {
+    hartree_fock(v, n, NQ, nao, jvec.get(), Kout.get() + (int64_t)i0 * nps * n2, nps, nj, stream);
+  });
   if (x2c) {
     // Ewald on the aa, bb, ab blocks with the AO overlap S_aa on both sides
     // (x2c_hf_gpu_kernel::add_Ewald, hf_gpu_kernel.cpp:304-327); ba follows
@@ -1858,9 +1848,7 @@ void HfPlan::solve(const double* dm, const double* S_k, double madelung, double*
   if (share_size > 1)
     for (int ik = 0; ik < sym.ink; ++ik)
       if (ik % share_size != share_rank) zero(Kout.get() + (int64_t)ik * nps * n2, (int64_t)nps * n2, stream);
-  energy_valid = false;
-  fetch(F);
-  compute_energy();
+  fetch(F, true);
 }
 
 }  // namespace ggpu

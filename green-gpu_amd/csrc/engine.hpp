@@ -343,11 +343,16 @@ struct HfPlan {
   // Kout[ik][s] from dm_fbz; the K partial sums of the split (k2, Q)
   // reduction go to `part` (nsp slices of nps nao^2)
   void exchange_device(z64* part, int nsp);
-  void fetch(double* out);  // Kout -> caller layout (ns, ink, nso, nso)
+  void to_caller_layout(z64* out);  // Kout -> (ns, ink, nso, nso) on the device
+  // Kout through F_dev to the host; with_energy: and the energy from
+  // dm_host_dev and those Fock matrices
+  void fetch(double* out, bool with_energy);
   std::vector<PairTable> diag_tables;  // (k, k) pairs: [0] all full k, [1] IBZ representatives
-  DeviceBuffer<z64> jvec, S_dev, Ftmp, dm2c_fbz, F2c, traces;
+  DeviceBuffer<z64> jvec, jpart, S_dev, Ftmp, dm2c_fbz, F_dev;
+  PinnedBuffer<z64> traces;   // Tr[D F] per (s, ik), written by the device
   DeviceBuffer<int64_t> kout_src, kout_dst;   // Kout (ik, s) -> caller layout (s, ik) slab offsets
-  void compute_energy();    // from dm_host_dev and the Fock matrices of solve()
+  void enqueue_traces();
+  void collect_energy();
   SpinorTables x2c_split, x2c_merge;
 };
 

@@ -133,14 +133,6 @@ __global__ void zero_int_kernel(int* p, int64_t n) {
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
     p[i] = 0;
 }
-__global__ void sum_partials_kernel(const z64* in, int64_t stride, int np, z64* out, int64_t n) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-    double re = 0.0, im = 0.0;
-    for (int p = 0; p < np; ++p) { const z64 v = in[p * stride + i]; re += v.x; im += v.y; }
-    out[i] = z64{re, im};
-  }
-}
-
 constexpr int NBMAX = 32;
 
 // One workgroup per matrix; the nb x nb diagonal block lives in LDS.
@@ -474,12 +466,6 @@ void zero(z64* p, int64_t n, hipStream_t s) {
 void zero_int(int* p, int64_t n, hipStream_t s) {
   if (n <= 0) return;
   hipLaunchKernelGGL(zero_int_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, p, n);
-  GGPU_HIP(hipGetLastError());
-}
-
-void sum_partials(const z64* in, int64_t stride, int np, z64* out, int64_t n, hipStream_t s) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(sum_partials_kernel, dim3(grid_for(n, 256)), dim3(256), 0, s, in, stride, np, out, n);
   GGPU_HIP(hipGetLastError());
 }
 

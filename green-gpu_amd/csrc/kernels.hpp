@@ -45,9 +45,6 @@ void to_c32(const z64* in, c32* out, int64_t n, hipStream_t s);
 void zero(z64* p, int64_t n, hipStream_t s);
 void zero_int(int* p, int64_t n, hipStream_t s);
 
-// out[i] = sum_p in[p * stride + i], i < n.
-void sum_partials(const z64* in, int64_t stride, int np, z64* out, int64_t n, hipStream_t s);
-
 // ---- batched blocked Cholesky (lower, A = L L^dagger), nw matrices n x n ----
 // Factor the nb x nb diagonal block at (j0, j0) in place; info[w] = column+1
 // of the first non-positive pivot (0 = fine).
