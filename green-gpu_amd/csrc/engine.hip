@@ -10,7 +10,6 @@
 //   work      pair-batch intermediates (X1, X2 for P0; Y1, Y2 for Sigma)
 #include "engine.hpp"
 #include "ozaki.hpp"
-#include "hf.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -1544,7 +1543,17 @@ HfPlan::HfPlan(int nao_, int nso_, int ns_, int NQ_, const ggpu_symmetry& s)
   // density block and slice) has about 1024 workgroups on the 256 CUs
   const int tiles = ((nao + 63) / 64) * ((nao + 63) / 64);
   nsplit = std::max(64, std::min(512, 1024 / (tiles * nps)));
-  Kpart.resize((size_t)nsplit * nps * n2);
+  int64_t part = (int64_t)nsplit * nps * n2;
+  if (exchange_fits(nao)) {
+    // partial K of every k at once, up to 256 MiB
+    ex_plan = exchange_plan(nao, NQ, nps, sym.nk, sym.ink, kb);
+    const int64_t per_k = (int64_t)ex_plan.slices * nps * n2;
+    part = std::max({part, per_k, std::min<int64_t>(per_k * sym.ink, (int64_t)16 << 20)});
+    std::vector<PairView> v;
+    for (const PairTable& t : tables) v.insert(v.end(), t.host.begin(), t.host.end());
+    all_pairs.build(v, stride, stream);
+  }
+  Kpart.resize((size_t)part);
   Kout.resize((size_t)sym.ink * nps * n2);
   jvec.resize(NQ);
   jpart.resize((size_t)sym.nk * NQ);
@@ -1628,7 +1637,55 @@ HfPlan::~HfPlan() {
 //   K[s][i][j]     += (px/nk) sum_{b,Q,c} X[s][b][Q][i][c] conj(V^Q(k,k2_b)[j][c])
 // The (b, Q) reduction is split into `nsplit` slices written to partial
 // buffers, so each launch has nsplit * ns workgroups instead of ns.
-void HfPlan::exchange_device(z64* kpart, int nsp) {
+void HfPlan::exchange_device(z64* kpart, int64_t part_cap) {
+  if (share_size > 1) zero(Kout.get(), Kout.size(), stream);
+  if (fused() && (int64_t)ex_plan.slices * nps * nao * nao <= part_cap)
+    exchange_fused(kpart, part_cap);
+  else
+    exchange_products(kpart, (int)std::max<int64_t>(1, std::min<int64_t>(nsplit, part_cap / ((int64_t)nps * nao * nao))));
+}
+
+// Whether the exchange runs the fused FP64 kernel: FP64 arithmetic at the HF
+// site (the int8 modes unless the caller forces the emulation) and a V^Q that
+// fits LDS three times.
+bool HfPlan::fused() const {
+  const int v = variants[kSiteHF];
+  return !complex64_operands(compute) && v != kVariantInt8 && v != kVariantInt8x5 && exchange_fits(nao);
+}
+
+// All k of this share in as few launches as the partial buffer allows when
+// the integrals are resident, per k and staged batch otherwise.
+void HfPlan::exchange_fused(z64* kpart, int64_t part_cap) {
+  const int64_t n2 = (int64_t)nao * nao, stride = (int64_t)NQ * n2;
+  const int64_t per_k = (int64_t)ex_plan.slices * nps * n2;
+  const double px = (nps == 1) ? -0.5 : -1.0;   // -1 for ns = 2 and the X2C blocks
+  const int nmine = share_rank < sym.ink ? (sym.ink - share_rank + share_size - 1) / share_size : 0;
+  const int group = store.staged() ? 1 : (int)std::max<int64_t>(1, std::min<int64_t>(part_cap / per_k, 65535));
+  for (int g0 = 0; g0 < nmine; g0 += group) {
+    const int ng = std::min(group, nmine - g0), ik = share_rank + g0 * share_size;
+    if (store.staged()) {
+      const int step = std::max(1, kb / ex_plan.per_chunk) * ex_plan.per_chunk;
+      for (int i0 = 0; i0 < sym.nk; i0 += step) {
+        const int n = std::min(step, sym.nk - i0);
+        const PairBlocks v = pair_blocks(store, tables[ik], i0, n, stride, stream);
+        exchange_f64(ex_plan, v, 0, 1, i0, n, nao, NQ, dm_fbz.get(), nps, px / sym.nk, kpart, stream);
+        store.done(stream);
+      }
+    } else {
+      const int64_t ld = (int64_t)share_size * sym.nk, last = (int64_t)ik * sym.nk + (ng - 1) * ld + sym.nk;
+      PairBlocks v = pair_blocks(store, all_pairs, 0, (int)last, stride, stream);
+      v.off += (int64_t)ik * sym.nk;
+      v.trans += (int64_t)ik * sym.nk;
+      v.conj += (int64_t)ik * sym.nk;
+      exchange_f64(ex_plan, v, (int)ld, ng, 0, sym.nk, nao, NQ, dm_fbz.get(), nps, px / sym.nk, kpart, stream);
+      store.done(stream);
+    }
+    sum_slices(kpart, per_k, (int64_t)nps * n2, ex_plan.slices, Kout.get() + (int64_t)ik * nps * n2,
+               (int64_t)share_size * nps * n2, (int64_t)nps * n2, ng, stream);
+  }
+}
+
+void HfPlan::exchange_products(z64* kpart, int nsp) {
   const int64_t n2 = (int64_t)nao * nao, stride = (int64_t)NQ * n2;
   const double px = (nps == 1) ? -0.5 : -1.0;   // -1 for ns = 2 and the X2C blocks
   const bool lp = complex64_operands(compute);
@@ -1644,7 +1701,6 @@ void HfPlan::exchange_device(z64* kpart, int nsp) {
   }
   const void* dm = lp ? (const void*)dm32.get() : (const void*)dm_fbz.get();
   const Span dsp{dm, dm_fbz.size()};
-  if (share_size > 1) zero(Kout.get(), Kout.size(), stream);
   const int64_t part_elems = (int64_t)nsp * nps * n2;
   for (int ik = share_rank; ik < sym.ink; ik += share_size) {
     zero(kpart, part_elems, stream);
@@ -1746,7 +1802,7 @@ void HfPlan::exchange(const double* dm, double* K) {
   require(dm && K, "hf: NULL pointer");
   GGPU_HIP(hipMemcpyAsync(dm_host_dev.get(), dm, dm_host_dev.bytes(), hipMemcpyHostToDevice, stream));
   stage_dm(dm_host_dev.get());
-  exchange_device(Kpart.get(), nsplit);
+  exchange_device(Kpart.get(), (int64_t)Kpart.size());
   fetch(K, false);
 }
 
@@ -1766,9 +1822,8 @@ void HfPlan::exchange_device_noalloc(const z64* dm_dev, z64* K_dev) {
           "hf no-alloc exchange: one partial slice of " + std::to_string(slice) +
               " complex elements exceeds the static scratch of " + std::to_string(scratch_elems));
   require(scratch == scratch_on_current_device(), "hf no-alloc exchange: plan created on another device");
-  const int nsp = (int)std::max<int64_t>(1, std::min<int64_t>(nsplit, scratch_elems / slice));
   stage_dm(dm_dev);
-  exchange_device(scratch, nsp);
+  exchange_device(scratch, scratch_elems);
   to_caller_layout(K_dev);
   GGPU_HIP(hipStreamSynchronize(stream));
 }
@@ -1782,7 +1837,7 @@ void HfPlan::solve(const double* dm, const double* S_k, double madelung, double*
   GGPU_HIP(hipMemcpyAsync(dm_host_dev.get(), dm, dm_host_dev.bytes(), hipMemcpyHostToDevice, stream));
   GGPU_HIP(hipMemcpyAsync(S_dev.get(), S_k, S_dev.bytes(), hipMemcpyHostToDevice, stream));
   stage_dm(dm_host_dev.get());
-  exchange_device(Kpart.get(), nsplit);                // Kout[ik][s]
+  exchange_device(Kpart.get(), (int64_t)Kpart.size());                // Kout[ik][s]
   // Hartree: jvec[Q] = (1/nk) sum_{k', s} sum_{a,b} V^Q(k',k')[a][b] D_s(k')[b][a]
   // (X2C: the density is D_aa + D_bb, blocks 0 and 1)
   const int nj = x2c ? 2 : ns;

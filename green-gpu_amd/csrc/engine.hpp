@@ -4,6 +4,7 @@
 
 #include "../../include/green_gpu_amd.h"
 #include "common.hpp"
+#include "hf.hpp"
 #include "kernels.hpp"
 #include "zgemm.hpp"
 
@@ -307,6 +308,8 @@ struct HfPlan {
   DeviceBuffer<z64> dm_host_dev, dm_fbz, Kpart, Kout, work;
   DeviceBuffer<int64_t> bidx_off;
   std::vector<PairTable> tables;   // per IBZ k: pairs (k, k2) for all k2
+  PairTable all_pairs;             // all of them, k after k (fused exchange)
+  ExchangePlan ex_plan;
   int kb = 1, nsplit = 1;
   // Arithmetic of the two exchange products (X = V D, K += X V^dagger); the
   // partial sums of K, J and the Ewald term are always FP64.
@@ -341,8 +344,11 @@ struct HfPlan {
  private:
   void stage_dm(const z64* dm_dev);   // caller-layout dm on the device -> dm_fbz (full BZ, density blocks)
   // Kout[ik][s] from dm_fbz; the K partial sums of the split (k2, Q)
-  // reduction go to `part` (nsp slices of nps nao^2)
-  void exchange_device(z64* part, int nsp);
+  // reduction go to `part` (part_cap elements, at least nps nao^2)
+  void exchange_device(z64* part, int64_t part_cap);
+  bool fused() const;
+  void exchange_fused(z64* part, int64_t part_cap);   // one kernel per group of k
+  void exchange_products(z64* part, int nsp);         // X = V D, K += X V^dagger as GEMMs, nsp slices
   void to_caller_layout(z64* out);  // Kout -> (ns, ink, nso, nso) on the device
   // Kout through F_dev to the host; with_energy: and the energy from
   // dm_host_dev and those Fock matrices

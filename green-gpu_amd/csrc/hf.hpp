@@ -1,4 +1,5 @@
-// Kernels of the Hartree term, the Fock assembly and the HF energy (hf.hip).
+// Kernels of the HF exchange (FP64), the Hartree term, the Fock assembly and the
+// HF energy (hf.hip).
 #pragma once
 
 #include "common.hpp"
@@ -14,6 +15,24 @@ struct PairBlocks {
   const int* trans = nullptr;     // device
   const int* conj = nullptr;      // device
 };
+
+// The fused FP64 exchange (nao that fits LDS): K_s(k) as `slices` partial
+// matrices, each summed over one chunk of the (k2, Q) entries.
+bool exchange_fits(int nao);
+struct ExchangePlan {
+  int per_chunk = 1;   // pairs per chunk (split == 1)
+  int split = 1;       // chunks per pair
+  int chunks = 0;      // of one k
+  int slices = 0;      // partial matrices of one k and density block
+};
+// kb: pairs a staged batch may hold (chunks never span batches of whole chunks).
+ExchangePlan exchange_plan(int nao, int NQ, int nps, int nk, int ink, int kb);
+// The chunks of pairs [b0, b0 + npairs) of `ngroup` k: pair b0 + b of group
+// entry g is v's entry g * pairs_ld + b.  b0 is a multiple of p.per_chunk, and
+// so is npairs unless the pairs end there.  D: (nk, nps, nao, nao);
+// part: (ngroup, p.slices, nps, nao, nao).
+void exchange_f64(const ExchangePlan& p, const PairBlocks& v, int pairs_ld, int ngroup, int b0, int npairs, int nao,
+                  int NQ, const z64* D, int nps, double scale, z64* part, hipStream_t s);
 
 // part[b * NQ + Q] = scale sum_{a,c} V_b^Q[a][c] sum_{s < nj} D[b][s][c][a]
 // for the n pairs b; D: (n, nps, nao, nao).
