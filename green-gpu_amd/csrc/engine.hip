@@ -29,6 +29,36 @@ static void gemm_on(GemmDesc g, const BA& a, const BB& b, const BC& c, hipStream
   gemm(g, s);
 }
 
+// One product per (pair, spin) entry e < count: A and B of entry e at element
+// offsets offA[fa + e] and offB[fb + e], C at e * c_step (es, ec: bytes per
+// element of the operands and of C).  Small products run as one batched
+// launch; large ones (their launches fill the chip by themselves) and the int8
+// emulation, whose workspace is sized per product, one by one.  The line is
+// about 0.3 ms of FP64 work: at nao = 26, NQ = 100 a launch per product is
+// 15 - 66 us, of which 5 - 8 us are its ramp and tail.
+template <class BA, class BB, class BC>
+static void gemm_entries(GemmDesc g, int count, const EntryOffsets& offA, int fa, const EntryOffsets& offB, int fb,
+                         int64_t c_step, int64_t es, int64_t ec, const BA& a, const BB& b, const BC& c,
+                         hipStream_t s) {
+  require(fa >= 0 && fa + count <= (int)offA.host.size() && fb >= 0 && fb + count <= (int)offB.host.size(),
+          "gw: entry offsets out of range");
+  if (count <= 65535 && gemm_flops(g) < 2e10 && !gemm_emulates_int8(g.compute, g.site)) {
+    g.nb1 = count;
+    g.A.off1 = offA.dev + fa; g.A.off1_host = offA.host.data() + fa;
+    g.B.off1 = offB.dev + fb; g.B.off1_host = offB.host.data() + fb;
+    g.C.bs1 = c_step;
+    gemm_on(g, a, b, c, s);
+    return;
+  }
+  for (int e = 0; e < count; ++e) {
+    GemmDesc h = g;
+    h.A.ptr = (const char*)g.A.ptr + offA.host[fa + e] * es;
+    h.B.ptr = (const char*)g.B.ptr + offB.host[fb + e] * es;
+    h.C.ptr = (char*)g.C.ptr + e * c_step * ec;
+    gemm_on(h, a, b, c, s);
+  }
+}
+
 // View of caller memory with a known element count (device pointers handed in).
 struct Span {
   const void* p;
@@ -667,8 +697,7 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
     GGPU_HIP(hipMemcpy(rev_src.get(), src.data(), src.size() * sizeof(int64_t), hipMemcpyHostToDevice));
     GGPU_HIP(hipMemcpy(rev_dst.get(), dst.data(), dst.size() * sizeof(int64_t), hipMemcpyHostToDevice));
   }
-  Sig_acc.resize((size_t)sym.ink * ns * nts * n2);
-  Sig_host_dev.resize(Sig_acc.size());
+  Sig_host_dev.resize((size_t)sym.ink * ns * nts * n2);
   P0.resize((size_t)p0_split * half * Q2);
   P0w.resize((size_t)nw_b * Q2);
   Amat.resize((size_t)nw_b * Q2);
@@ -730,6 +759,69 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
   for (int b = 0; b < kb; ++b) bo[b] = b * stride;
   bidx_off.resize(kb);
   GGPU_HIP(hipMemcpy(bidx_off.get(), bo.data(), bo.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+
+  // per-entry operand offsets of the batched small products
+  const int64_t gs = (int64_t)nts * n2;   // G of one (k, spin)
+  auto spins = [&](const std::vector<int64_t>& first, int64_t step) {
+    std::vector<int64_t> v;
+    for (int64_t f : first)
+      for (int s2 = 0; s2 < ns; ++s2) v.push_back(f + s2 * step);
+    return v;
+  };
+  v_entries.host = spins(bo, 0);
+  p_entries.host.assign((size_t)kb * ns, 0);
+  for (int e = 0; e < kb * ns; ++e) y_entries.host.push_back((int64_t)e * nts * stride);
+  p0_g.resize(sym.inq);
+  p0_grev.resize(sym.inq);
+  sig_g.resize(sym.inq);
+  for (int iq = 0; iq < sym.inq; ++iq) {
+    std::vector<int64_t> k0, k1;
+    for (int ik = 0; ik < sym.ink; ++ik)
+      for (auto k : sym.k_stars[ik]) {
+        k0.push_back(k * ns * gs);
+        k1.push_back(sym.k1_from_k2q[k * sym.nq + sym.q_r2f[iq]] * ns * gs);
+      }
+    p0_grev[iq].host = spins(k0, gs);
+    p0_g[iq].host = spins(k1, gs);
+    sig_g[iq].resize(sym.q_stars[iq].size());
+    for (size_t j = 0; j < sym.q_stars[iq].size(); ++j) {
+      std::vector<int64_t> k2;
+      for (int ik = 0; ik < sym.ink; ++ik)
+        k2.push_back(sym.k2_from_k1q[sym.k_r2f[ik] * sym.nq + sym.q_stars[iq][j]] * ns * gs);
+      sig_g[iq][j].host = spins(k2, gs);
+    }
+  }
+  {
+    std::vector<EntryOffsets*> all = {&v_entries, &p_entries, &y_entries};
+    for (int iq = 0; iq < sym.inq; ++iq) {
+      all.push_back(&p0_grev[iq]);
+      all.push_back(&p0_g[iq]);
+      for (auto& t : sig_g[iq]) all.push_back(&t);
+    }
+    std::vector<int64_t> flat;
+    for (auto* t : all) flat.insert(flat.end(), t->host.begin(), t->host.end());
+    entry_offsets.resize(flat.size());
+    GGPU_HIP(hipMemcpy(entry_offsets.get(), flat.data(), flat.size() * sizeof(int64_t), hipMemcpyHostToDevice));
+    size_t at = 0;
+    for (auto* t : all) {
+      t->dev = entry_offsets.get() + at;
+      at += t->host.size();
+    }
+  }
+  if (!lowp()) {
+    // with up to two 64 x 32 tiles per CU in a Sigma contraction launch, slices
+    // of at least 8 auxiliary functions for about four per CU: nk = 1, nao = 10,
+    // NQ = 154 (two-component) 168 -> 60 us; above that the gain is under 2 %
+    // (the complex64 modes keep one FP32 sum over all Q)
+    const int64_t sig = (int64_t)Sig_host_dev.size();
+    const int64_t tiles = (int64_t)((nts * nao + 63) / 64) * ((nao + 31) / 32) * ns * std::min(kb, sym.ink);
+    const int64_t split = tiles > 512 ? 1 : std::min<int64_t>({(1024 + tiles - 1) / tiles, NQ / 8, ((int64_t)1 << 26) / sig});
+    if (split > 1) {
+      const int len = (int)((NQ + split - 1) / split);
+      sig_split = (NQ + len - 1) / len;
+    }
+  }
+  Sig_acc.resize((size_t)sig_split * Sig_host_dev.size());
 
   if (x2c) {
     // G: rotated spinor slabs (k, t) -> pseudo-spin blocks (k, ss, t);
@@ -798,16 +890,11 @@ void GwPlan::stage_G(const z64* G_dev) {
 void GwPlan::p0_for_q(int iq) {
   const int64_t n2 = (int64_t)nao * nao, stride = (int64_t)NQ * n2;
   const PairTable& tab = p0_tables[iq];
-  const int64_t q = sym.q_r2f[iq];
   const int npairs = (int)tab.host.size();
   const double pref = (ns == 1) ? -2.0 : -1.0;
   const bool lp = lowp();
   const int64_t es = lp ? (int64_t)sizeof(c32) : (int64_t)sizeof(z64);
   zero(P0.get(), (int64_t)P0.size(), stream);
-  // full-BZ k of every pair, in table order
-  std::vector<int64_t> ks;
-  for (int ik = 0; ik < sym.ink; ++ik)
-    for (auto k : sym.k_stars[ik]) ks.push_back(k);
   char* Vdir = reinterpret_cast<char*>(work.get());
   char* VpmQ = Vdir + kb * stride * es;
   char* X1 = VpmQ + kb * stride * es;
@@ -826,28 +913,23 @@ void GwPlan::p0_for_q(int iq) {
     tr.rows = (int)n2; tr.cols = NQ; tr.in_ld = n2; tr.out_ld = NQ;
     tr.n_inner = n; tr.in_bs = stride; tr.out_bs = stride; tr.trans_all = 1;
     block_copy(tr, stream);
-    for (int b = 0; b < n; ++b) {
-      const int64_t k = ks[i0 + b], k1 = sym.k1_from_k2q[k * sym.nq + q];
-      for (int s = 0; s < ns; ++s) {
-        // rows (t, n) of the tau-reversed G: one tall GEMM for all t < nts/2
-        GemmDesc g;
-        g.compute = compute; g.out_f32 = lp;
-        g.M = half * nao; g.N = nao * NQ; g.K = nao;
-        g.A.ptr = (const char*)Gr + (k * ns + s) * nts * n2 * es; g.A.rs = nao; g.A.cs = 1;
-        g.B.ptr = VpmQ + b * stride * es; g.B.rs = (int64_t)nao * NQ; g.B.cs = 1;
-        g.C.ptr = X1 + (b * ns + s) * xs * es; g.C.rs = (int64_t)nao * NQ; g.C.cs = 1;
-        g.site = kSiteP0X1;
-        gemm_on(g, grsp, wk, wk, stream);
-        GemmDesc h;
-        h.compute = compute; h.out_f32 = lp;
-        h.M = NQ * nao; h.N = nao; h.K = nao; h.nb0 = half;
-        h.A.ptr = Vdir + b * stride * es; h.A.rs = nao; h.A.cs = 1; h.A.conj = 1;
-        h.B.ptr = (const char*)Gp + (k1 * ns + s) * nts * n2 * es; h.B.rs = 1; h.B.cs = nao; h.B.bs0 = n2;
-        h.C.ptr = X2 + (b * ns + s) * xs * es; h.C.rs = nao; h.C.cs = 1; h.C.bs0 = stride;
-        h.site = kSiteP0X2;
-        gemm_on(h, wk, gsp, wk, stream);
-      }
-    }
+    // rows (t, n) of the tau-reversed G: one tall GEMM for all t < nts/2
+    GemmDesc g;
+    g.compute = compute; g.out_f32 = lp;
+    g.M = half * nao; g.N = nao * NQ; g.K = nao;
+    g.A.ptr = Gr; g.A.rs = nao; g.A.cs = 1;
+    g.B.ptr = VpmQ; g.B.rs = (int64_t)nao * NQ; g.B.cs = 1;
+    g.C.ptr = X1; g.C.rs = (int64_t)nao * NQ; g.C.cs = 1;
+    g.site = kSiteP0X1;
+    gemm_entries(g, n * ns, p0_grev[iq], i0 * ns, v_entries, 0, xs, es, es, grsp, wk, wk, stream);
+    GemmDesc h;
+    h.compute = compute; h.out_f32 = lp;
+    h.M = NQ * nao; h.N = nao; h.K = nao; h.nb0 = half;
+    h.A.ptr = Vdir; h.A.rs = nao; h.A.cs = 1; h.A.conj = 1;
+    h.B.ptr = Gp; h.B.rs = 1; h.B.cs = nao; h.B.bs0 = n2;
+    h.C.ptr = X2; h.C.rs = nao; h.C.cs = 1; h.C.bs0 = stride;
+    h.site = kSiteP0X2;
+    gemm_entries(h, n * ns, v_entries, 0, p0_g[iq], i0 * ns, xs, es, es, wk, gsp, wk, stream);
     // P0 partial slice j accumulates (pair, spin) entries j, j + S, j + 2S, ...
     // (FP64 partials also in the reduced-precision modes)
     const int E = n * ns, S = p0_split, full = E / S, rem = E - full * S;
@@ -1069,28 +1151,22 @@ void GwPlan::sigma_for_q(int iq) {
     for (int i0 = 0; i0 < sig_end; i0 += kb) {
       const int n = std::min(kb, sym.ink - i0);
       unfold_pairs(store, tab, i0, n, bidx_off.get(), Vdir, lp, NQ, nao, stream);
-      for (int b = 0; b < n; ++b) {
-        const int64_t k = sym.k_r2f[i0 + b];
-        const int64_t k1 = sym.k2_from_k1q[k * sym.nq + qd];
-        for (int s = 0; s < ns; ++s) {
-          GemmDesc g;
-          g.compute = compute; g.out_f32 = lp;
-          g.M = NQ * nao; g.N = nao; g.K = nao; g.nb0 = nts;
-          g.A.ptr = Vdir + b * stride * es; g.A.rs = nao; g.A.cs = 1;
-          g.B.ptr = (const char*)Gp + (k1 * ns + s) * nts * n2 * es; g.B.rs = nao; g.B.cs = 1; g.B.bs0 = n2;
-          g.C.ptr = Y1 + (b * ns + s) * ys * es; g.C.rs = nao; g.C.cs = 1; g.C.bs0 = stride;
-          g.site = kSiteSigY1;
-          gemm_on(g, wk, gsp, wk, stream);
-          GemmDesc h;
-          h.compute = compute; h.out_f32 = lp;
-          h.M = NQ; h.N = (int)n2; h.K = NQ; h.nb0 = nts;
-          h.A.ptr = Pq; h.A.rs = 1; h.A.cs = NQ; h.A.bs0 = Q2; h.A.conj = tr;
-          h.B.ptr = Y1 + (b * ns + s) * ys * es; h.B.rs = n2; h.B.cs = 1; h.B.bs0 = stride;
-          h.C.ptr = Y2 + (b * ns + s) * ys * es; h.C.rs = (int64_t)nts * n2; h.C.cs = 1; h.C.bs0 = n2;
-          h.site = kSiteSigY2;
-          gemm_on(h, psp, wk, wk, stream);
-        }
-      }
+      GemmDesc g;
+      g.compute = compute; g.out_f32 = lp;
+      g.M = NQ * nao; g.N = nao; g.K = nao; g.nb0 = nts;
+      g.A.ptr = Vdir; g.A.rs = nao; g.A.cs = 1;
+      g.B.ptr = Gp; g.B.rs = nao; g.B.cs = 1; g.B.bs0 = n2;
+      g.C.ptr = Y1; g.C.rs = nao; g.C.cs = 1; g.C.bs0 = stride;
+      g.site = kSiteSigY1;
+      gemm_entries(g, n * ns, v_entries, 0, sig_g[iq][j], i0 * ns, ys, es, es, wk, gsp, wk, stream);
+      GemmDesc h;
+      h.compute = compute; h.out_f32 = lp;
+      h.M = NQ; h.N = (int)n2; h.K = NQ; h.nb0 = nts;
+      h.A.ptr = Pq; h.A.rs = 1; h.A.cs = NQ; h.A.bs0 = Q2; h.A.conj = tr;
+      h.B.ptr = Y1; h.B.rs = n2; h.B.cs = 1; h.B.bs0 = stride;
+      h.C.ptr = Y2; h.C.rs = (int64_t)nts * n2; h.C.cs = 1; h.C.bs0 = n2;
+      h.site = kSiteSigY2;
+      gemm_entries(h, n * ns, p_entries, 0, y_entries, 0, ys, es, es, psp, wk, wk, stream);
       GemmDesc f;
       f.compute = compute; f.out_f32 = 0;       // Sigma accumulates in FP64
       f.M = nts * nao; f.N = nao; f.K = nao; f.KB = NQ; f.nb0 = n; f.nb1 = ns;
@@ -1100,6 +1176,14 @@ void GwPlan::sigma_for_q(int iq) {
       f.C.bs0 = (int64_t)ns * nts * n2; f.C.bs1 = (int64_t)nts * n2;
       f.alpha_re = -1.0; f.beta_re = 1.0;
       f.site = kSiteSigma;
+      if (sig_split > 1 && !gemm_emulates_int8(compute, kSiteSigma)) {
+        // slices of the Q sum, one accumulator each
+        const int64_t sig = (int64_t)sym.ink * ns * nts * n2;
+        f.KB = (NQ + sig_split - 1) / sig_split; f.kb_total = NQ; f.nb0 = sig_split; f.nb1 = n * ns;
+        f.A.bs0 = f.KB * f.A.kbs; f.A.bs1 = ys;
+        f.B.bs0 = f.KB * f.B.kbs; f.B.off1 = v_entries.dev; f.B.off1_host = v_entries.host.data();
+        f.C.bs0 = sig; f.C.bs1 = (int64_t)nts * n2;
+      }
       gemm_on(f, wk, wk, Sig_acc, stream);
     }
   }
@@ -1228,6 +1312,10 @@ void GwPlan::enqueue_iteration(const z64* G_dev, z64* S_dev, bool timed) {
     if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 3], stream));
   }
   if (timed) GGPU_HIP(hipEventRecord(ev[5], stream));
+  if (sig_split > 1) {
+    const int64_t sig = (int64_t)Sig_acc.size() / sig_split;
+    sum_slices(Sig_acc.get(), 0, sig, sig_split, Sig_acc.get(), 0, sig, 1, stream);
+  }
   if (x2c)
     spinor_copy(x2c_merge, Sig_acc.get(), Sig_acc.size(), nao, n2, S_dev, Sig_host_dev.size(), nso,
                 (int64_t)sym.ink * nso * nso, nao, nts, 1.0 / sym.nk, stream);

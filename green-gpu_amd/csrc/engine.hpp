@@ -172,6 +172,13 @@ struct SpinorTables {
              const std::vector<int>& cj);
 };
 
+// Element offsets of the (pair, spin) entries of a chain: the device table of
+// a batched launch and its host copy.
+struct EntryOffsets {
+  const int64_t* dev = nullptr;         // in GwPlan::entry_offsets
+  std::vector<int64_t> host;
+};
+
 struct GwPlan {
   // ns: spin blocks the contractions run over (the two-component plan runs
   // over the four pseudo-spins aa, bb, ab, ba); nso: size of the caller's
@@ -201,6 +208,14 @@ struct GwPlan {
   DeviceBuffer<char> ozwork;            // slices and scales of the int8-emulated FP64 products
   DeviceBuffer<int64_t> bidx_off;       // b * NQ * nao^2
   DeviceBuffer<int64_t> sig_src, sig_dst;
+  DeviceBuffer<int64_t> entry_offsets;  // the device copies of the tables below
+  EntryOffsets v_entries;               // entry e = b * ns + s of a pair batch: b * NQ * nao^2
+  EntryOffsets p_entries, y_entries;    // 0 (one P for all) and e * nts * NQ * nao^2
+  std::vector<EntryOffsets> p0_g, p0_grev;          // per IBZ q: G(k + q) and G(k) of every entry
+  std::vector<std::vector<EntryOffsets>> sig_g;     // per IBZ q, per star member: G(k - q)
+  // Sigma accumulators (slices of the Q sum): more workgroups per contraction
+  // launch where (pairs, spins, tau rows) leave the chip idle
+  int sig_split = 1;
   std::vector<PairTable> p0_tables;     // per IBZ q
   std::vector<std::vector<PairTable>> sig_tables;  // per IBZ q, per star member
   FullBZRotator rot;

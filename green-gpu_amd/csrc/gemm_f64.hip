@@ -93,7 +93,8 @@ __global__ __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(WP
   }
   const char *Ab = reinterpret_cast<const char*>(A), *Bb = reinterpret_cast<const char*>(B);   // of a K-batch entry
   const int64_t a_kb = d.A.kbs * 16, b_kb = d.B.kbs * 16, a_kt = d.A.cs * (16 * BK), b_kt = d.B.rs * (16 * BK);
-  const int ktiles = (d.K + BK - 1) / BK, niter = d.KB * ktiles;
+  const int nkb = d.kb_total > 0 ? min(d.KB, d.kb_total - (int)tc.b0 * d.KB) : d.KB;
+  const int ktiles = (d.K + BK - 1) / BK, niter = nkb * ktiles;
   const int tail = d.K - (ktiles - 1) * BK;   // k extent of a K-batch entry's last tile
   const char *pa = Ab, *pb = Bb;
   int ikt = 0;                                // tile (pa, pb) point at

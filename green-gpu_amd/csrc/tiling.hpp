@@ -18,22 +18,21 @@ __device__ inline int64_t xcd_logical(int64_t id, int64_t total) {
 }
 
 // Logical tile -> (m-tile, n-tile, batch b0, batch b1).  Default order:
-// m-tile fastest, then n-tile, then batch.  With d.batch_major the batch
-// index runs fastest instead: chosen when every batch shares A (A's batch
-// strides are zero), so the workgroups reusing one A panel run back to back
-// and find it in L2 instead of re-reading A from memory once per batch.
+// m-tile fastest, then n-tile, then batch b1, then b0.  With d.batch_major b0
+// runs fastest and b1 slowest: chosen when every b0 shares A, so the
+// workgroups reusing one A panel run back to back and find it in L2 instead of
+// re-reading A from memory once per batch.
 struct TileCoord { int mt, nt; int64_t b0, b1; };
 __device__ inline TileCoord tile_coord(const GemmDesc& d, int tiles_m, int tiles_n) {
   int64_t lg = xcd_logical(blockIdx.x, gridDim.x);
   TileCoord c;
   if (d.batch_major) {
-    const int64_t nb = (int64_t)d.nb0 * d.nb1;
-    const int64_t b = lg % nb;
-    lg /= nb;
+    c.b0 = lg % d.nb0;
+    lg /= d.nb0;
     c.mt = (int)(lg % tiles_m);
-    c.nt = (int)(lg / tiles_m);
-    c.b1 = b % d.nb1;
-    c.b0 = b / d.nb1;
+    lg /= tiles_m;
+    c.nt = (int)(lg % tiles_n);
+    c.b1 = lg / tiles_n;
   } else {
     c.mt = (int)(lg % tiles_m);
     lg /= tiles_m;

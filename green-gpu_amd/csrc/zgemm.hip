@@ -1210,10 +1210,16 @@ void gemm_check_bounds(const GemmDesc& d) {
   require(d.nb0 <= 65535 && d.nb1 <= 65535, "gemm: batch count above 65535");
   if (d.M == 0 || d.N == 0) return;
   Range ra, rb, rc;
-  extend(ra, d.M, d.A.rs); extend(ra, d.K, d.A.cs); extend(ra, d.KB, d.A.kbs);
-  extend(ra, d.nb0, d.A.bs0); if (!d.A.off1) extend(ra, d.nb1, d.A.bs1);
-  extend(rb, d.K, d.B.rs); extend(rb, d.N, d.B.cs); extend(rb, d.KB, d.B.kbs);
-  extend(rb, d.nb0, d.B.bs0); if (!d.B.off1) extend(rb, d.nb1, d.B.bs1);
+  if (d.kb_total > 0)
+    require(d.compute != Compute::F32 && d.compute != Compute::BF16X3 && (int64_t)d.KB * d.nb0 >= d.kb_total &&
+                (int64_t)d.KB * (d.nb0 - 1) < d.kb_total && d.A.bs0 == d.KB * d.A.kbs && d.B.bs0 == d.KB * d.B.kbs,
+            "gemm: bad slices of the K-batch");
+  const int64_t entries = d.kb_total > 0 ? d.kb_total : d.KB;
+  const int nb0 = d.kb_total > 0 ? 1 : d.nb0;   // of the operands
+  extend(ra, d.M, d.A.rs); extend(ra, d.K, d.A.cs); extend(ra, entries, d.A.kbs);
+  extend(ra, nb0, d.A.bs0); if (!d.A.off1) extend(ra, d.nb1, d.A.bs1);
+  extend(rb, d.K, d.B.rs); extend(rb, d.N, d.B.cs); extend(rb, entries, d.B.kbs);
+  extend(rb, nb0, d.B.bs0); if (!d.B.off1) extend(rb, d.nb1, d.B.bs1);
   extend(rc, d.M, d.C.rs); extend(rc, d.N, d.C.cs);
   extend(rc, d.nb0, d.C.bs0); if (!d.C.off1) extend(rc, d.nb1, d.C.bs1);
   const size_t ein = complex64_operands(d.compute) ? sizeof(float2) : sizeof(double2);
@@ -1263,11 +1269,17 @@ bool gemm_variant_valid(Compute c, int v) {
   return std::find(cand, cand + n, v) != cand + n;
 }
 
+bool gemm_emulates_int8(Compute c, int site) {
+  if (!int8_slices(c)) return false;
+  const int v = (g_site_variants && site >= 0 && site < kNumSites) ? g_site_variants[site] : -1;
+  return v == kVariantInt8 || v == kVariantInt8x5 || (v == -1 && (site == kSiteSigY2 || site == kSiteP0));
+}
+
 void gemm(const GemmDesc& dd, hipStream_t stream) {
   gemm_check_bounds(dd);
   if (dd.M == 0 || dd.N == 0) return;
   GemmDesc d = dd;
-  d.batch_major = (d.nb0 * (int64_t)d.nb1 > 1) && d.A.bs0 == 0 && d.A.bs1 == 0 && d.A.off1 == nullptr;
+  d.batch_major = d.nb0 > 1 && d.A.bs0 == 0;
   const int v = (g_site_variants && d.site >= 0 && d.site < kNumSites) ? g_site_variants[d.site] : -1;
   if (g_profiler) g_profiler->before(d, stream);
   switch (d.compute) {
@@ -1285,9 +1297,8 @@ void gemm(const GemmDesc& dd, hipStream_t stream) {
       break;
     case Compute::I8X5:
     case Compute::I8X4: {
-      const bool emulate =
-          v == kVariantInt8 || v == kVariantInt8x5 || (v == -1 && (d.site == kSiteSigY2 || d.site == kSiteP0));
-      if (emulate) {
+      if (gemm_emulates_int8(d.compute, d.site)) {
+        require(d.kb_total == 0, "gemm: the int8 emulation takes no K-batch slices");
         gemm_int8_emulated(d, v == kVariantInt8x5 ? 5 : int8_slices(d.compute), g_workspace, g_workspace_bytes,
                            stream);
       } else {

@@ -136,8 +136,12 @@ inline bool int8_site_tunable(Compute c, int site, int variant = kVariantInt8) {
 
 struct GemmDesc {
   int site = kSiteOther;
-  int batch_major = 0;   // set by gemm(): batch index fastest in the tile order
+  int batch_major = 0;   // set by gemm(): batch index b0 fastest in the tile order
   int M = 0, N = 0, K = 0, KB = 1;
+  // FP64 only, > 0: batch b0 is one of nb0 slices of a sum over kb_total K-batch
+  // entries, KB of them (the last slice has the rest); the operands' bs0 are
+  // KB kbs.
+  int kb_total = 0;
   int nb0 = 1, nb1 = 1;
   Operand A, B;
   OutOperand C;
@@ -146,6 +150,10 @@ struct GemmDesc {
   Compute compute = Compute::F64;
   int out_f32 = 0;             // C holds complex64 (only with F32 / BF16X3 compute)
 };
+
+// Whether a launch of this compute mode at this site runs the int8 emulation
+// (the calling thread's launch variants, else the built-in choice).
+bool gemm_emulates_int8(Compute c, int site);
 
 // Throws Error(kErrArgument) if any address the launch would touch falls
 // outside an operand's declared allocation.
@@ -161,7 +169,8 @@ void gemm(const GemmDesc& d, hipStream_t stream);
 
 // Algorithmic FLOPs of the launch: 8 per complex multiply-add.
 inline double gemm_flops(const GemmDesc& d) {
-  return 8.0 * d.M * (double)d.N * d.K * d.KB * d.nb0 * d.nb1;
+  const double entries = d.kb_total > 0 ? d.kb_total : (double)d.KB * d.nb0;
+  return 8.0 * d.M * (double)d.N * d.K * entries * d.nb1;
 }
 
 }  // namespace ggpu
