@@ -368,17 +368,32 @@ __device__ inline void split2(float a, float b, unsigned& hi, unsigned& lo) {
   lo = __builtin_bit_cast(unsigned, __builtin_convertvector(v2f{a - ha, b - hb}, v2bf));
   hi = h;
 }
+//
+// The vector unit bounds it next to the matrix pipe (120 MFMAs per 32 k and
+// wave of a 160 x 64 tile take as long as 480 vector instructions), so the
+// loader has nothing per element: one 32-bit offset per group of eight, the
+// eight k by uniform pointers, rows past the edge clamped (they are never
+// stored) and k past the end, in an entry's last tile only, clamped by one
+// select and zeroed before the split.  Bounds and 64-bit addresses for each
+// element cost 550 vector instructions and 32 branches per 32 k, more than the
+// matrix products.  At nao = 52, NQ = 300, nts = 110 (one q, 16 pair-spins;
+// before -> after): sig_py 15.5 -> 13.8 ms, p0_contract 7.6 -> 6.9, sig_contract
+// 5.9 -> 4.4, p0_gvh 2.8 -> 2.4.  Every site takes as long as its matrix and
+// vector instructions one after the other: the two waves of a SIMD meet at the
+// same barriers.
+constexpr int XROWS = 160;   // most rows or columns of a tile
 
 template <class TO, bool AKC, bool BKC, int WMB, int WNB, int SITE, int WPE = 1>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_bf16x3_big_kernel(
     const GemmDesc d) {
   constexpr int TM = 32 * WMB, TN = 32 * WNB, LDK = XBK + XPAD;
+  static_assert(TM <= XROWS && TN <= XROWS && TM * 4 % 64 == 0 && TN * 4 % 64 == 0, "tile");
   constexpr int GA = (TM * 4 + NTHREADS - 1) / NTHREADS;   // 8-element groups per thread
   constexpr int GB = (TN * 4 + NTHREADS - 1) / NTHREADS;
   __shared__ __attribute__((aligned(16))) unsigned short sA[4][TM][LDK];
   __shared__ __attribute__((aligned(16))) unsigned short sB[4][TN][LDK];
 
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tiles_m = (d.M + TM - 1) / TM;
   const int tiles_n = (d.N + TN - 1) / TN;
   const TileCoord tc = tile_coord(d, tiles_m, tiles_n);
@@ -388,69 +403,95 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
   const float2* B = static_cast<const float2*>(d.B.ptr) + b0 * d.B.bs0 + (d.B.off1 ? d.B.off1[b1] : b1 * d.B.bs1);
   TO* C = static_cast<TO*>(d.C.ptr) + b0 * d.C.bs0 + (d.C.off1 ? d.C.off1[b1] : b1 * d.C.bs1);
 
+  // Group u of a thread: its row and first k.  Waves without a group of their
+  // own load the last one again and do not store it.  k0u: the wave has one k0.
+  constexpr bool A_K0U = !AKC && TM % 64 == 0, B_K0U = !BKC && TN % 64 == 0;
+  auto has = [&](int u, int rows) { return wave * 64 + u * NTHREADS < rows * 4; };
+  const uint32_t a_ks = AKC ? 8u : (uint32_t)d.A.cs * 8u, b_ks = BKC ? 8u : (uint32_t)d.B.rs * 8u;
   int arow[GA], ak0[GA], brow[GB], bk0[GB];
+  uint32_t ar0[GA], av[GA], br0[GB], bv[GB];   // byte offset of the group's row, of its first element
 #pragma unroll
   for (int u = 0; u < GA; ++u) {
-    const int g = tid + u * NTHREADS;
+    const int g = min(wave + u * (NTHREADS / 64), TM / 16 - 1) * 64 + (tid & 63);
     arow[u] = AKC ? (g >> 2) : (g % TM);
     ak0[u] = AKC ? ((g & 3) << 3) : ((g / TM) << 3);
-    if (g >= TM * 4) arow[u] = -1;
+    if (A_K0U) ak0[u] = __builtin_amdgcn_readfirstlane(ak0[u]);
+    ar0[u] = (uint32_t)min(arow[u], d.M - 1 - m0) * (uint32_t)(d.A.rs * 8);
+    av[u] = ar0[u] + (uint32_t)ak0[u] * a_ks;
   }
 #pragma unroll
   for (int u = 0; u < GB; ++u) {
-    const int g = tid + u * NTHREADS;
+    const int g = min(wave + u * (NTHREADS / 64), TN / 16 - 1) * 64 + (tid & 63);
     brow[u] = BKC ? (g >> 2) : (g % TN);
     bk0[u] = BKC ? ((g & 3) << 3) : ((g / TN) << 3);
-    if (g >= TN * 4) brow[u] = -1;
+    if (B_K0U) bk0[u] = __builtin_amdgcn_readfirstlane(bk0[u]);
+    br0[u] = (uint32_t)min(brow[u], d.N - 1 - n0) * (uint32_t)(d.B.cs * 8);
+    bv[u] = br0[u] + (uint32_t)bk0[u] * b_ks;
   }
   const int ktiles = (d.K + XBK - 1) / XBK;
   const int niter = d.KB * ktiles;
+  const int tail = d.K - (ktiles - 1) * XBK;   // k extent of a K-batch entry's last tile
+  const char *Ab = reinterpret_cast<const char*>(A + (int64_t)m0 * d.A.rs),
+             *Bb = reinterpret_cast<const char*>(B + (int64_t)n0 * d.B.cs);
+  const int64_t a_kb = d.A.kbs * 8, b_kb = d.B.kbs * 8;
+  const char *pa = Ab, *pb = Bb;
+  int ikt = 0;                                 // tile (pa, pb) point at
   float2 ra[GA][8], rb[GB][8];
-  auto gload = [&](int it) {
-    const int kb = it / ktiles;
-    const int kt = (it - kb * ktiles) * XBK;
-    const float2* Ab = A + kb * d.A.kbs;
-    const float2* Bb = B + kb * d.B.kbs;
+  // a k past the end reads another k of the row
+  auto load8 = [&](float2 (&x)[8], const char* p, bool k0u, uint32_t ks, uint32_t v, uint32_t r0, int k0, int rem) {
 #pragma unroll
-    for (int u = 0; u < GA; ++u) {
-      const int gm = m0 + arow[u];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int gk = kt + ak0[u] + j;
-        ra[u][j] = (arow[u] >= 0 && gm < d.M && gk < d.K) ? Ab[gm * d.A.rs + gk * d.A.cs] : float2{0.f, 0.f};
-      }
+    for (int j = 0; j < 8; ++j) {
+      if (k0u) x[j] = *reinterpret_cast<const float2*>(p + (uint32_t)min(k0 + j, rem - 1) * ks + r0);
+      else x[j] = *reinterpret_cast<const float2*>(p + (uint32_t)min(j, rem - 1) * ks + (k0 + j < rem ? v : r0));
     }
+  };
+  auto gload = [&]() {
+    const int rem = ikt + 1 == ktiles ? tail : XBK;
 #pragma unroll
-    for (int u = 0; u < GB; ++u) {
-      const int gn = n0 + brow[u];
+    for (int u = 0; u < GA; ++u) load8(ra[u], pa, A_K0U, a_ks, av[u], ar0[u], ak0[u], rem);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int gk = kt + bk0[u] + j;
-        rb[u][j] = (brow[u] >= 0 && gn < d.N && gk < d.K) ? Bb[gk * d.B.rs + gn * d.B.cs] : float2{0.f, 0.f};
-      }
+    for (int u = 0; u < GB; ++u) load8(rb[u], pb, B_K0U, b_ks, bv[u], br0[u], bk0[u], rem);
+    pa += (int64_t)XBK * a_ks;
+    pb += (int64_t)XBK * b_ks;
+    if (++ikt == ktiles) {
+      ikt = 0;
+      pa = Ab += a_kb;
+      pb = Bb += b_kb;
     }
   };
   // split 8 consecutive-k elements into the re_hi, im_hi, re_lo, im_lo planes
-  auto split8 = [&](unsigned short (*S)[LDK], int rows, int row, int k0, const float2* x, bool conj) {
-    unsigned hr[4], hi[4], lr_[4], li[4];
+  auto split8 = [&](unsigned short (*S)[LDK], int rows, int row, int k0, const float2* x, bool conj, int rem) {
+    unsigned p[4][4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-      const float s = conj ? -1.f : 1.f;
-      split2(x[2 * q].x, x[2 * q + 1].x, hr[q], lr_[q]);
-      split2(s * x[2 * q].y, s * x[2 * q + 1].y, hi[q], li[q]);
+      split2(x[2 * q].x, x[2 * q + 1].x, p[0][q], p[2][q]);
+      split2(x[2 * q].y, x[2 * q + 1].y, p[1][q], p[3][q]);
     }
-    *reinterpret_cast<v4u*>(&S[0 * rows + row][k0]) = v4u{hr[0], hr[1], hr[2], hr[3]};
-    *reinterpret_cast<v4u*>(&S[1 * rows + row][k0]) = v4u{hi[0], hi[1], hi[2], hi[3]};
-    *reinterpret_cast<v4u*>(&S[2 * rows + row][k0]) = v4u{lr_[0], lr_[1], lr_[2], lr_[3]};
-    *reinterpret_cast<v4u*>(&S[3 * rows + row][k0]) = v4u{li[0], li[1], li[2], li[3]};
+    if (conj)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        p[1][q] ^= 0x80008000u;
+        p[3][q] ^= 0x80008000u;
+      }
+    if (rem < XBK)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int k = k0 + 2 * q;
+        const unsigned m = k + 1 < rem ? ~0u : k < rem ? 0xffffu : 0u;
+#pragma unroll
+        for (int pl = 0; pl < 4; ++pl) p[pl][q] &= m;
+      }
+#pragma unroll
+    for (int pl = 0; pl < 4; ++pl)
+      *reinterpret_cast<v4u*>(&S[pl * rows + row][k0]) = v4u{p[pl][0], p[pl][1], p[pl][2], p[pl][3]};
   };
-  auto sstore = [&]() {
+  auto sstore = [&](int rem) {
 #pragma unroll
     for (int u = 0; u < GA; ++u)
-      if (arow[u] >= 0) split8(&sA[0][0], TM, arow[u], ak0[u], ra[u], d.A.conj != 0);
+      if (has(u, TM)) split8(&sA[0][0], TM, arow[u], ak0[u], ra[u], d.A.conj != 0, rem);
 #pragma unroll
     for (int u = 0; u < GB; ++u)
-      if (brow[u] >= 0) split8(&sB[0][0], TN, brow[u], bk0[u], rb[u], d.B.conj != 0);
+      if (has(u, TN)) split8(&sB[0][0], TN, brow[u], bk0[u], rb[u], d.B.conj != 0, rem);
   };
 
   const int lane = tid & 63, w = tid >> 6;
@@ -463,11 +504,12 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
     for (int j = 0; j < WNB; ++j) { cr[i][j] = v4f{0, 0, 0, 0}; ci[i][j] = v4f{0, 0, 0, 0}; }
   const v4u sign = v4u{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
 
-  if (niter > 0) gload(0);
-  for (int it = 0; it < niter; ++it) {
-    sstore();
+  if (niter > 0) gload();
+  for (int it = 0, kt = 0; it < niter; ++it) {
+    sstore(kt + 1 == ktiles ? tail : XBK);
+    if (++kt == ktiles) kt = 0;
     __syncthreads();
-    if (it + 1 < niter) gload(it + 1);
+    if (it + 1 < niter) gload();
     v8bf brh[WNB], bih[WNB], brl[WNB], bil[WNB];
 #pragma unroll
     for (int j = 0; j < WNB; ++j) {
@@ -1027,84 +1069,9 @@ void launch_bf16x3_astat(const GemmDesc& d, hipStream_t stream) {
   GGPU_HIP(hipGetLastError());
 }
 
-template <class TO, int WMB, int WNB, int SITE, int WPE = 1>
-void launch_bf16x3_big(const GemmDesc& d, hipStream_t stream) {
-  constexpr int TM = 32 * WMB, TN = 32 * WNB;
-  const int64_t tiles = (int64_t)((d.M + TM - 1) / TM) * ((d.N + TN - 1) / TN);
-  const int64_t total = tiles * d.nb0 * d.nb1;
-  require(total < (int64_t)1 << 31, "gemm: grid too large");
-  dim3 grid((unsigned)total), block(NTHREADS);
-  const bool akc = (d.A.cs == 1) || (d.A.rs != 1);
-  const bool bkc = (d.B.rs == 1) || (d.B.cs != 1);
-  if (akc && bkc)
-    hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, true, true, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
-  else if (akc)
-    hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, true, false, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
-  else if (bkc)
-    hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, false, true, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
-  else
-    hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, false, false, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
-  GGPU_HIP(hipGetLastError());
-}
-
-// Fraction of a tiled extent that is real work.
-inline double tile_use(int n, int t) { return (double)n / (double)(((n + t - 1) / t) * t); }
-
+// 64 x 64 tiles with 64-bit addresses: any strides.
 template <class TO, int SITE>
-void launch_bf16x3_site(const GemmDesc& d, hipStream_t stream, int variant) {
-  int mode = variant;
-  if (mode < 0) {
-    // Two or three waves per SIMD (6- to 10-block wave tiles) beat bigger
-    // tiles.  Large shapes take the tile measured fastest for their call site
-    // inside a GW iteration on MI355X (nao = 52, NQ = 300, nts = 110; every
-    // tile forced in turn, per-launch times from the site profiler) unless
-    // its tile waste is more than 10 % above the best fit of the two-wave
-    // tiles; other shapes take that best fit.  (Repeated launches of one GEMM
-    // on the same operands rank the tiles differently: warm caches.)
-    mode = kBf16Tile64x64;
-    if (d.M >= 64 && d.N >= 48 && (d.M >= 128 || d.N >= 128)) {
-      const int cand[5] = {kBf16Tile128x64, kBf16Tile64x128, kBf16Tile160x64, kBf16Tile96x64W3, kBf16Tile64x64W3};
-      const double use[5] = {tile_use(d.M, 128) * tile_use(d.N, 64), tile_use(d.M, 64) * tile_use(d.N, 128),
-                             tile_use(d.M, 160) * tile_use(d.N, 64), tile_use(d.M, 96) * tile_use(d.N, 64),
-                             tile_use(d.M, 64) * tile_use(d.N, 64)};
-      int best = 0;
-      for (int c = 1; c < 3; ++c)
-        if (use[c] > use[best] + 0.03) best = c;
-      int pref = -1;
-      switch (SITE) {
-        case kSiteSigY1: case kSiteSigma: pref = 0; break;   // 128 x 64
-        case kSiteSigY2: pref = 1; break;                    // 64 x 128
-        case kSiteP0X2: case kSiteP0: pref = 2; break;       // 160 x 64
-        case kSiteP0X1: pref = 3; break;                     // 96 x 64, three waves
-        default: break;
-      }
-      mode = cand[(pref >= 0 && use[pref] >= 0.9 * use[best]) ? pref : best];
-    }
-  }
-  switch (mode) {
-    case kBf16Tile128x64: return launch_bf16x3_big<TO, 4, 2, SITE>(d, stream);
-    case kBf16Tile64x128: return launch_bf16x3_big<TO, 2, 4, SITE>(d, stream);
-    case kBf16Tile160x64: return launch_bf16x3_big<TO, 5, 2, SITE>(d, stream);
-    case kBf16Tile96x64W3: return launch_bf16x3_big<TO, 3, 2, SITE, 3>(d, stream);
-    case kBf16Tile64x96W3: return launch_bf16x3_big<TO, 2, 3, SITE, 3>(d, stream);
-    case kBf16Tile64x64W3: return launch_bf16x3_big<TO, 2, 2, SITE, 3>(d, stream);
-    case kBf16TileAstat64x64:
-      if (astat_fits(d)) return launch_bf16x3_astat<TO, SITE>(d, stream);
-      return launch_bf16x3_big<TO, 2, 2, SITE, 3>(d, stream);   // a 64 x 64 tile, A staged per batch
-    case kBf16TileFrag128x128:
-      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 2, 2>(d, stream);
-      return launch_bf16x3_big<TO, 5, 2, SITE>(d, stream);   // no workspace: 160 x 64
-    case kBf16TileFrag128x128W8:
-      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 4, 2>(d, stream);
-      return launch_bf16x3_big<TO, 5, 2, SITE>(d, stream);
-    case kBf16TileFrag128x128W16:
-      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 4, 4>(d, stream);
-      return launch_bf16x3_big<TO, 5, 2, SITE>(d, stream);
-    case kBf16TileFrag128x192W8:
-      if (fb_fits(d, 192)) return launch_bf16x3_frag<TO, 2, 4, 192>(d, stream);
-      return launch_bf16x3_big<TO, 5, 2, SITE>(d, stream);
-    default: break;
-  }
+void launch_bf16x3_64(const GemmDesc& d, hipStream_t stream) {
   const int64_t tiles = (int64_t)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN);
   const int64_t total = tiles * d.nb0 * d.nb1;
   require(total < (int64_t)1 << 31, "gemm: grid too large");
@@ -1116,6 +1083,110 @@ void launch_bf16x3_site(const GemmDesc& d, hipStream_t stream, int variant) {
   else if (bkc) hipLaunchKernelGGL((gemm_bf16x3_kernel<TO, false, true, SITE>), grid, block, 0, stream, d);
   else hipLaunchKernelGGL((gemm_bf16x3_kernel<TO, false, false, SITE>), grid, block, 0, stream, d);
   GGPU_HIP(hipGetLastError());
+}
+
+// Lane offsets of the big kernel are 32 bits wide; what reaches further, or
+// backwards, takes the 64 x 64 kernel with 64-bit addresses.
+bool big_tiles_fit(const GemmDesc& d) {
+  auto span = [](int64_t rs, int64_t ks) { return 8.0 * (XROWS * (double)rs + XBK * (double)ks); };
+  return d.A.rs >= 0 && d.A.cs >= 0 && d.B.rs >= 0 && d.B.cs >= 0 && span(d.A.rs, d.A.cs) < 4294967296.0 &&
+         span(d.B.cs, d.B.rs) < 4294967296.0;
+}
+
+// Layout a call site compiles for (its own symbol); another one runs as
+// kSiteOther.
+constexpr bool site_akc(int site) { return site != kSiteP0 && site != kSiteSigY2; }
+constexpr bool site_bkc(int site) { return site == kSiteP0X2 || site == kSiteP0 || site == kSiteSigma; }
+
+template <class TO, int WMB, int WNB, int SITE, int WPE = 1>
+void launch_bf16x3_big(const GemmDesc& d, hipStream_t stream) {
+  constexpr int TM = 32 * WMB, TN = 32 * WNB;
+  if (!big_tiles_fit(d)) return launch_bf16x3_64<TO, SITE>(d, stream);
+  const int64_t tiles = (int64_t)((d.M + TM - 1) / TM) * ((d.N + TN - 1) / TN);
+  const int64_t total = tiles * d.nb0 * d.nb1;
+  require(total < (int64_t)1 << 31, "gemm: grid too large");
+  dim3 grid((unsigned)total), block(NTHREADS);
+  const bool akc = d.A.cs == 1, bkc = d.B.rs == 1;
+  if constexpr (SITE != kSiteOther) {
+    if (akc == site_akc(SITE) && bkc == site_bkc(SITE)) {
+      hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, site_akc(SITE), site_bkc(SITE), WMB, WNB, SITE, WPE>), grid, block,
+                         0, stream, d);
+      GGPU_HIP(hipGetLastError());
+      return;
+    }
+    launch_bf16x3_big<TO, WMB, WNB, kSiteOther, WPE>(d, stream);
+  } else {
+    if (akc && bkc)
+      hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, true, true, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
+    else if (akc)
+      hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, true, false, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
+    else if (bkc)
+      hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, false, true, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
+    else
+      hipLaunchKernelGGL((gemm_bf16x3_big_kernel<TO, false, false, WMB, WNB, SITE, WPE>), grid, block, 0, stream, d);
+    GGPU_HIP(hipGetLastError());
+  }
+}
+
+// Fraction of a tiled extent that is real work.
+inline double tile_use(int n, int t) { return (double)n / (double)(((n + t - 1) / t) * t); }
+
+template <class TO, int SITE>
+void launch_bf16x3_site(const GemmDesc& d, hipStream_t stream, int variant) {
+  int mode = variant;
+  if (mode < 0) {
+    // The tile that wastes least, except that each call site's fastest tile of
+    // a full grid is taken while it wastes at most 10 % more (nao = 52, NQ = 300,
+    // every tile forced in turn: sig_py 160 x 64 13.8 ms, others 14.2-16.2;
+    // p0_contract 160 x 64 6.9, others 7.7-8.9; sig_contract 128 x 64 4.4, others
+    // 4.5-7.1; sig_vg 64 x 64 with A kept 4.3, others 4.8-8.4).  128 x 32 does 0.8 of
+    // the work per area: for N <= 32 and the like.  A GW iteration with this
+    // rule against 64 x 64 at every site, nao = 12 to 104: 0-5 % faster at
+    // all nine sizes but one (nao = 90: 2 % slower).
+    struct Tile { int mode, m, n; };
+    constexpr Tile cand[] = {{kBf16Tile128x64, 128, 64}, {kBf16Tile64x128, 64, 128}, {kBf16Tile160x64, 160, 64},
+                             {kBf16Tile96x64W3, 96, 64}, {kBf16Tile64x64W3, 64, 64}, {kBf16Tile128x32, 128, 32}};
+    constexpr int n_cand = sizeof(cand) / sizeof(cand[0]);
+    const int pref = SITE == kSiteP0X1 || SITE == kSiteP0X2 || SITE == kSiteP0 || SITE == kSiteSigY2 ? 2
+                     : SITE == kSiteSigY1 || SITE == kSiteSigma ? 0 : -1;
+    double use[n_cand];
+    int best = 0;
+    for (int c = 0; c < n_cand; ++c) {
+      use[c] = tile_use(d.M, cand[c].m) * tile_use(d.N, cand[c].n) * (cand[c].mode == kBf16Tile128x32 ? 0.8 : 1.0);
+      if (use[c] > use[best] + 0.03) best = c;
+    }
+    if (pref >= 0 && use[pref] >= 0.9 * use[best]) best = pref;
+    mode = cand[best].mode;
+    // too few of them for the chip: more, smaller ones
+    if ((int64_t)((d.M + cand[best].m - 1) / cand[best].m) * ((d.N + cand[best].n - 1) / cand[best].n) * d.nb0 * d.nb1 < 512)
+      mode = kBf16Tile64x64W3;
+    if (SITE == kSiteSigY1 && mode == kBf16Tile128x64 && astat_fits(d)) mode = kBf16TileAstat64x64;
+  }
+  switch (mode) {
+    case kBf16Tile128x64: return launch_bf16x3_big<TO, 4, 2, SITE, 2>(d, stream);
+    case kBf16Tile64x128: return launch_bf16x3_big<TO, 2, 4, SITE, 2>(d, stream);
+    case kBf16Tile160x64: return launch_bf16x3_big<TO, 5, 2, SITE, 2>(d, stream);
+    case kBf16Tile96x64W3: return launch_bf16x3_big<TO, 3, 2, SITE, 3>(d, stream);
+    case kBf16Tile64x96W3: return launch_bf16x3_big<TO, 2, 3, SITE, 3>(d, stream);
+    case kBf16Tile64x64W3: return launch_bf16x3_big<TO, 2, 2, SITE, 3>(d, stream);
+    case kBf16Tile128x32: return launch_bf16x3_big<TO, 4, 1, SITE, 3>(d, stream);
+    case kBf16TileAstat64x64:
+      if (astat_fits(d)) return launch_bf16x3_astat<TO, SITE>(d, stream);
+      return launch_bf16x3_big<TO, 2, 2, SITE, 3>(d, stream);   // a 64 x 64 tile, A staged per batch
+    case kBf16TileFrag128x128:
+      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 2, 2>(d, stream);
+      return launch_bf16x3_big<TO, 5, 2, SITE, 2>(d, stream);   // no workspace: 160 x 64
+    case kBf16TileFrag128x128W8:
+      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 4, 2>(d, stream);
+      return launch_bf16x3_big<TO, 5, 2, SITE, 2>(d, stream);
+    case kBf16TileFrag128x128W16:
+      if (fb_fits(d, 128)) return launch_bf16x3_frag<TO, 4, 4>(d, stream);
+      return launch_bf16x3_big<TO, 5, 2, SITE, 2>(d, stream);
+    case kBf16TileFrag128x192W8:
+      if (fb_fits(d, 192)) return launch_bf16x3_frag<TO, 2, 4, 192>(d, stream);
+      return launch_bf16x3_big<TO, 5, 2, SITE, 2>(d, stream);
+    default: return launch_bf16x3_64<TO, SITE>(d, stream);
+  }
 }
 
 template <class TO>
