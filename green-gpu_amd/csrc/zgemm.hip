@@ -1,27 +1,13 @@
-// Batched complex GEMM on the gfx950 matrix cores.
+// Batched complex GEMM on the gfx950 matrix cores: the dispatch of every compute
+// mode, and the split-bf16 kernels (FP64 and FP32 have their own files).
 //
-// The dispatch of every compute mode, and the FP32 and split-bf16 kernels (FP64
-// has its own file).
-//
-// FP32 workgroup = 4 wave64s computing a 64 x 64 complex tile of C; each wave
-// owns a 32 x 32 quadrant = 2 x 2 blocks of the 16 x 16 MFMA output, kept as
-// separate real / imaginary accumulators (4 real MFMAs per complex block and
-// k-step: re += ar*br - ai*bi, im += ar*bi + ai*br).
-//
-// Tiles of A (64 x 16) and B (16 x 64) are staged through LDS as split
-// real / imaginary planes, k-major, so the MFMA operand reads (lane -> row
-// lane%16, k lane/16) are unit-stride across 16 lanes.  The next tile is
-// prefetched from global memory into registers while the current one is
-// multiplied.  Global loads follow whichever operand dimension is contiguous
-// (template flags), so every operand layout of the HF/GW chains streams with
-// full 64-byte segments.
-//
-// Split-bf16 x3 has its own kernels further down: tiles from 64 x 64 to
-// 160 x 64 that split complex64 operands into bf16 hi / lo planes while
-// staging them, and an A-stationary 64 x 64 tile that splits one shared A
-// once and walks several batches.  Each call site is its own kernel symbol;
-// the launch variant per site comes from the built-in choice, a per-thread
-// table (the plan's autotuned choice) or a global override.
+// Split-bf16 x3 tiles from 64 x 64 to 160 x 64 split complex64 operands into
+// bf16 hi / lo planes while staging them; an A-stationary 64 x 64 tile splits
+// one shared A once and walks several batches.  Global loads follow whichever
+// operand dimension is contiguous (template flags), so every operand layout of
+// the HF/GW chains streams with full 64-byte segments.  Each call site is its
+// own kernel symbol; the launch variant per site comes from the built-in
+// choice, a per-thread table (the plan's autotuned choice) or a global override.
 #include "tiling.hpp"
 #include "ozaki.hpp"
 
@@ -33,161 +19,12 @@ namespace {
 
 constexpr int BM = 64;
 constexpr int BN = 64;
-constexpr int BKT = 16;
 constexpr int NTHREADS = 256;
-constexpr int PAD = 2;
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // Row (within the 16 x 16 block) of accumulator register r of lane group
 // lk = lane / 16 is 4 lk + r, the column lane % 16 (measured on gfx950).
-// FP32 kernel.  TO: complex element type of C.
-// AKC: A's k index is the contiguous one (else its m index).
-// BKC: B's k index is the contiguous one (else its n index).
-// 4 real products per complex product.
-// BK: k per LDS stage (16, or 8 for half the LDS and twice the workgroups
-// per CU).
-// WPE: waves per SIMD the register allocation must allow (1: no constraint).
-template <class TO, bool AKC, bool BKC, int SITE, int BK = BKT, int WPE = 1>
-__global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE))) void gemm_mfma_kernel(
-    const GemmDesc d) {
-  using T = float;
-  using CT = c32;
-  using AV = v4f;
-  constexpr int EPT = BM * BK / NTHREADS;   // complex elements per thread and operand
-  __shared__ T sA[2][2][BK][BM + PAD];   // [buffer][re/im][k][m]
-  __shared__ T sB[2][2][BK][BN + PAD];   // [buffer][re/im][k][n]
-
-  const int tid = threadIdx.x;
-  const int tiles_m = (d.M + BM - 1) / BM;
-  const int tiles_n = (d.N + BN - 1) / BN;
-  const TileCoord tc = tile_coord(d, tiles_m, tiles_n);
-  const int m0 = tc.mt * BM, n0 = tc.nt * BN;
-  const int64_t b1 = tc.b1, b0 = tc.b0;
-
-  const CT* A = static_cast<const CT*>(d.A.ptr) + b0 * d.A.bs0 + (d.A.off1 ? d.A.off1[b1] : b1 * d.A.bs1);
-  const CT* B = static_cast<const CT*>(d.B.ptr) + b0 * d.B.bs0 + (d.B.off1 ? d.B.off1[b1] : b1 * d.B.bs1);
-  TO* C = static_cast<TO*>(d.C.ptr) + b0 * d.C.bs0 + (d.C.off1 ? d.C.off1[b1] : b1 * d.C.bs1);
-
-  // Loader coordinates inside the tile: EPT consecutive complex elements per
-  // thread along the operand's contiguous index.
-  constexpr int TK = BK / EPT, TMN = BM / EPT;   // threads per k-row / per m-row
-  int a_m[EPT], a_k[EPT], b_k[EPT], b_n[EPT];
-#pragma unroll
-  for (int j = 0; j < EPT; ++j) {
-    if (AKC) { a_m[j] = tid / TK; a_k[j] = (tid % TK) * EPT + j; }
-    else     { a_k[j] = tid / TMN; a_m[j] = (tid % TMN) * EPT + j; }
-    if (BKC) { b_n[j] = tid / TK; b_k[j] = (tid % TK) * EPT + j; }
-    else     { b_k[j] = tid / TMN; b_n[j] = (tid % TMN) * EPT + j; }
-  }
-
-  const int ktiles = (d.K + BK - 1) / BK;
-  const int niter = d.KB * ktiles;
-  CT ra[EPT], rb[EPT];
-
-  auto gload = [&](int it, CT (&xa)[EPT], CT (&xb)[EPT]) {
-    const int kb = it / ktiles;
-    const int k0 = (it - kb * ktiles) * BK;
-    const CT* Ab = A + kb * d.A.kbs;
-    const CT* Bb = B + kb * d.B.kbs;
-#pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      const int gm = m0 + a_m[j], gk = k0 + a_k[j];
-      xa[j] = (gm < d.M && gk < d.K) ? Ab[gm * d.A.rs + gk * d.A.cs] : CT{0, 0};
-      const int gk2 = k0 + b_k[j], gn = n0 + b_n[j];
-      xb[j] = (gk2 < d.K && gn < d.N) ? Bb[gk2 * d.B.rs + gn * d.B.cs] : CT{0, 0};
-    }
-  };
-  auto sstore = [&](int buf, const CT (&xa)[EPT], const CT (&xb)[EPT]) {
-#pragma unroll
-    for (int j = 0; j < EPT; ++j) {
-      sA[buf][0][a_k[j]][a_m[j]] = xa[j].x;
-      sA[buf][1][a_k[j]][a_m[j]] = d.A.conj ? -xa[j].y : xa[j].y;
-      sB[buf][0][b_k[j]][b_n[j]] = xb[j].x;
-      sB[buf][1][b_k[j]][b_n[j]] = d.B.conj ? -xb[j].y : xb[j].y;
-    }
-  };
-
-  const int lane = tid & 63, w = tid >> 6;
-  const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-  const int lr = lane & 15, lk = lane >> 4;
-  AV acc[2][2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[a][i][j] = AV{0, 0, 0, 0};
-
-  // One k-step of 4: fragments from LDS, then the block products.
-  auto kstep = [&](int buf, int kk) {
-    T ar[2], ai[2], br[2], bi[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      ar[i] = sA[buf][0][kk + lk][wm + 16 * i + lr];
-      ai[i] = sA[buf][1][kk + lk][wm + 16 * i + lr];
-      br[i] = sB[buf][0][kk + lk][wn + 16 * i + lr];
-      bi[i] = sB[buf][1][kk + lk][wn + 16 * i + lr];
-    }
-    T nai[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) nai[i] = -ai[i];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[i], br[j], acc[0][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ar[i], bi[j], acc[1][i][j], 0, 0, 0);
-        acc[0][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(nai[i], bi[j], acc[0][i][j], 0, 0, 0);
-        acc[1][i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(ai[i], br[j], acc[1][i][j], 0, 0, 0);
-      }
-  };
-
-  // All k-steps of k-tile it (LDS buffer it & 1).
-  auto ksteps = [&](int it) {
-    const int buf = it & 1;
-    const int k0 = (it % ktiles) * BK;
-#pragma unroll
-    for (int kk = 0; kk < BK; kk += 4)
-      if (k0 + kk < d.K) kstep(buf, kk);   // uniform: skip steps past the end of K
-  };
-
-  if (niter > 0) {
-    gload(0, ra, rb);
-    sstore(0, ra, rb);
-  }
-  __syncthreads();
-  for (int it = 0; it < niter; ++it) {
-    if (it + 1 < niter) gload(it + 1, ra, rb);   // next k-tile, into registers
-    ksteps(it);
-    if (it + 1 < niter) sstore((it & 1) ^ 1, ra, rb);
-    __syncthreads();
-  }
-
-  const bool use_beta = (d.beta_re != 0.0 || d.beta_im != 0.0);
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + 16 * i + 4 * lk + r;
-        const int col = n0 + wn + 16 * j + lr;
-        if (row < d.M && col < d.N) {
-          const double xr = acc[0][i][j][r], xi = acc[1][i][j][r];
-          double vr = d.alpha_re * xr - d.alpha_im * xi;
-          double vi = d.alpha_re * xi + d.alpha_im * xr;
-          TO* p = C + row * d.C.rs + col * d.C.cs;
-          if (use_beta) {
-            const TO o = *p;
-            vr += d.beta_re * o.x - d.beta_im * o.y;
-            vi += d.beta_re * o.y + d.beta_im * o.x;
-          }
-          using TS = decltype(TO{}.x);
-          *p = TO{static_cast<TS>(vr), static_cast<TS>(vi)};
-        }
-      }
-}
 
 // ---------------------------------------------------------------------------
 // Split-bf16 x3 kernel.  Operands are complex64 in memory; every element x is
@@ -1202,50 +1039,6 @@ void launch_bf16x3(const GemmDesc& d, hipStream_t stream, int v) {
   }
 }
 
-template <class TO, int SITE, int BK, int WPE>
-void launch_f32_bk(const GemmDesc& d, hipStream_t stream) {
-  const int64_t tiles = (int64_t)((d.M + BM - 1) / BM) * ((d.N + BN - 1) / BN);
-  const int64_t total = tiles * d.nb0 * d.nb1;
-  require(total < (int64_t)1 << 31, "gemm: grid too large");
-  dim3 grid((unsigned)total), block(NTHREADS);
-  const bool akc = (d.A.cs == 1) || (d.A.rs != 1);
-  const bool bkc = (d.B.rs == 1) || (d.B.cs != 1);
-  if (akc && bkc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, true, true, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else if (akc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, true, false, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else if (bkc) hipLaunchKernelGGL((gemm_mfma_kernel<TO, false, true, SITE, BK, WPE>), grid, block, 0, stream, d);
-  else hipLaunchKernelGGL((gemm_mfma_kernel<TO, false, false, SITE, BK, WPE>), grid, block, 0, stream, d);
-  GGPU_HIP(hipGetLastError());
-}
-
-template <class TO, int SITE>
-void launch_f32_site(const GemmDesc& d, hipStream_t stream, int variant) {
-  // Variants measured on MI355X (nao = 52, NQ = 300, nts = 110; medians of
-  // interleaved rounds): staging 8 k per LDS step is faster than 16 or equal
-  // at every call site; FP32 runs five waves unconstrained.  All variants give
-  // the same sums bit for bit.
-  switch (variant > 0 ? variant : 8) {
-    case 8: return launch_f32_bk<TO, SITE, 8, 1>(d, stream);
-    case 83: return launch_f32_bk<TO, SITE, 8, 3>(d, stream);
-    default: return launch_f32_bk<TO, SITE, 16, 1>(d, stream);
-  }
-}
-
-// FP32 keeps 4 products per complex product (the Gauss recombination
-// t3 - t1 - t2 of the FP64 kernel loses relative accuracy when the result is
-// small against |A||B|, which FP32 cannot afford).
-template <class TO>
-void launch_f32(const GemmDesc& d, hipStream_t stream, int v) {
-  switch (d.site) {
-    case kSiteP0X1: launch_f32_site<TO, kSiteP0X1>(d, stream, v); break;
-    case kSiteP0X2: launch_f32_site<TO, kSiteP0X2>(d, stream, v); break;
-    case kSiteP0: launch_f32_site<TO, kSiteP0>(d, stream, v); break;
-    case kSiteSigY1: launch_f32_site<TO, kSiteSigY1>(d, stream, v); break;
-    case kSiteSigY2: launch_f32_site<TO, kSiteSigY2>(d, stream, v); break;
-    case kSiteSigma: launch_f32_site<TO, kSiteSigma>(d, stream, v); break;
-    default: launch_f32_site<TO, kSiteOther>(d, stream, v); break;
-  }
-}
-
 // Range of element offsets (relative to ptr) touched by a 2-D view with the
 // given extents and strides, over all batch indices.
 struct Range { int64_t lo = 0, hi = 0; };
@@ -1359,8 +1152,7 @@ void gemm(const GemmDesc& dd, hipStream_t stream) {
       launch_f64(d, stream, v);
       break;
     case Compute::F32:
-      if (d.out_f32) launch_f32<float2>(d, stream, v);
-      else launch_f32<double2>(d, stream, v);
+      launch_f32(d, stream, v);
       break;
     case Compute::BF16X3:
       if (d.out_f32) launch_bf16x3<float2>(d, stream, v);

@@ -165,6 +165,9 @@ void gemm_check_bounds(const GemmDesc& d);
 // picks for the shape.
 void launch_f64(const GemmDesc& d, hipStream_t stream, int variant);
 
+// The same for FP32; variant 8: the 64 x 64 tile, 16: the 128 x 64 tile.
+void launch_f32(const GemmDesc& d, hipStream_t stream, int variant);
+
 // Enqueue the GEMM on `stream`.
 void gemm(const GemmDesc& d, hipStream_t stream);
 
