@@ -12,10 +12,9 @@
 // leave an error of about 2^-(7 NSL - 1) of max|A_m| max|B_n| per term of the
 // k sum: 2^-34 with five slices (FP64-accurate products for the contractions
 // here), 2^-27 with four.
-// Complex products use four real products per slice pair; the negated
-// imaginary slice of A is formed in registers (bytewise), so re and im
-// accumulate exactly:
-//   re += Ar_s Br_t + (-Ai_s) Bi_t,   im += Ar_s Bi_t + Ai_s Br_t.
+// Complex products use four real products per slice pair, in three
+// accumulators, so that no operand has to be negated:
+//   rr += Ar_s Br_t,  ii += Ai_s Bi_t,  im += Ar_s Bi_t + Ai_s Br_t,  re = rr - ii.
 //
 // Slices are stored fragment-native: for every (batch, k block of 64, block
 // of 16 rows, plane) one 1 KiB fragment whose lane l holds row l % 16 and the
@@ -401,28 +400,25 @@ __device__ inline void oz_store(const OzGemm& g, int64_t b0, int64_t b1, int row
   *C = out;
 }
 
-// Bytewise two's-complement negation of 16 packed int8 digits (|digit| <= 127).
-__device__ inline v4i neg_bytes(v4i x) {
-  v4i r;
-#pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const unsigned int n = ~(unsigned int)x[c];
-    r[c] = (int)(((n & 0x7f7f7f7fu) + 0x01010101u) ^ (n & 0x80808080u));
-  }
-  return r;
-}
-
 __device__ inline v4i lds_frag(const int8_t* p) { return *reinterpret_cast<const v4i*>(p); }
 
-// One 64 x 64 output tile per workgroup, 2 x WNW waves of 32 x (64 / WNW)
-// (2 x 4 / WNW blocks of the 16 x 16 MFMA output): four waves of 32 x 32,
-// one per SIMD, or eight of 32 x 16, two per SIMD.  Both operands'
-// fragments of a k block (80 KiB) are copied HBM -> LDS by the load-to-LDS
-// path into one of two stages while the other stage is multiplied, one
-// barrier per k block.
-// Within a k block every wave walks its A slices from the last to the first,
-// so the B fragments it needs grow by one slice per step and are read from
-// LDS one step ahead of their first use.
+// The 64 x 64 output tile of a workgroup: eight waves of 32 x 16 (2 x 1 blocks
+// of the 16 x 16 MFMA output), two per SIMD.  Both operands' fragments of a k
+// block (80 KiB with five slices) are copied HBM -> LDS by the load-to-LDS path
+// into one of two stages while the other stage is multiplied, one barrier
+// per k block.
+//
+// What bounds it (M = 600, N = 10816, K = 600, 110 batches, four slices): MFMAs
+// 10.5 ms, copies by themselves 13.5 ms, of 20 ms in all, at the 2.0 - 2.1 GHz
+// that the power draw allows (2.35 without the copies).  Vector instructions
+// between the MFMAs count too: negating A's imaginary slices in registers (96
+// a wave and k block) cost 0.8 ms, which the third accumulator saves: 25.2 -> 24.3
+// ms with the slicing, p0_contract 29.6 -> 28.5, sig_contract 18.0 -> 16.9,
+// five slices 32.6 -> 31.1, 37.4 -> 35.2, 21.0 -> 20.5.  Three real products per
+// complex one (balanced digits, sums formed in registers) need a quarter fewer
+// MFMAs but 192 vector instructions, and gave the same time; a 128 x 64 tile on
+// a ring of five 32 KiB chunks, with waits by count and a quarter fewer bytes
+// copied, gained 4 % here and lost 3 - 13 % elsewhere.
 //
 // Tile order: workgroups are dispatched round-robin over the 8 XCDs; the
 // linear id is remapped so every XCD works on a contiguous range of tiles,
@@ -430,108 +426,101 @@ __device__ inline v4i lds_frag(const int8_t* p) { return *reinterpret_cast<const
 // column, so the ~32 tiles an XCD runs at once cover GM row panels of A (kept
 // in its L2 while the group sweeps the columns) and ~32 / GM column panels of B.
 constexpr int GM = 4;
+constexpr int GEMM_WAVES = 8, GEMM_WN = 4;   // waves; waves along the columns
 
-template <class TO, int NSL, int WNW>
-__global__ __launch_bounds__(128 * WNW) void oz_gemm_kernel(const OzGemm g) {
-  constexpr int DMAX = NSL, NP = 2 * NSL, STAGE = stage_bytes<NSL>(), STAGE_A = STAGE / 2;
-  constexpr int NW = 2 * WNW, RJ = 4 / WNW;   // waves; column blocks per wave (2 row blocks each)
-  __shared__ __attribute__((aligned(1024))) int8_t lds[2 * STAGE];
-  const int tiles_m = (g.M + TILE - 1) / TILE, tiles_n = (g.N + TILE - 1) / TILE;
-  int64_t L = oz_xcd_logical(blockIdx.x, gridDim.x);
-  int mt, nt;
-  int64_t b0, b1;
+// Coordinates of logical tile L: within a batch, groups of GM row tiles,
+// column after column (or the batch index fastest when every batch shares A).
+struct OzTile {
+  int m0, n0;
+  int64_t b0, b1, bA, bB;
+};
+__device__ inline OzTile oz_tile(const OzGemm& g, int64_t tile, int tiles_m, int tiles_n) {
+  unsigned L = (unsigned)tile;   // a launch has fewer than 2^31 tiles
+  unsigned mt, nt, bb;
   if (g.batch_major) {
-    const int64_t nb = (int64_t)g.nb0 * g.nb1, bb = L % nb;
+    const unsigned nb = (unsigned)g.nb0 * (unsigned)g.nb1;
+    bb = L % nb;
     L /= nb;
-    mt = (int)(L % tiles_m);
-    nt = (int)(L / tiles_m);
-    b1 = bb % g.nb1;
-    b0 = bb / g.nb1;
+    mt = L % (unsigned)tiles_m;
+    nt = L / (unsigned)tiles_m;
   } else {
-    const int per_batch = tiles_m * tiles_n;
-    const int64_t bb = L / per_batch;
-    const int r = (int)(L - bb * per_batch);
-    const int mg = r / (GM * tiles_n), rem = r - mg * (GM * tiles_n);
-    const int gm = min(GM, tiles_m - mg * GM);   // row tiles in this group
+    const unsigned per_batch = (unsigned)tiles_m * (unsigned)tiles_n, span = GM * (unsigned)tiles_n;
+    bb = L / per_batch;
+    const unsigned r = L - bb * per_batch, mg = r / span, rem = r - mg * span;
+    const unsigned gm = min((unsigned)GM, (unsigned)tiles_m - mg * GM);   // row tiles in this group
     nt = rem / gm;
     mt = mg * GM + (rem - nt * gm);
-    b1 = bb % g.nb1;
-    b0 = bb / g.nb1;
   }
-  const int m0 = mt * TILE, n0 = nt * TILE;
-  const int64_t bA = g.a_shared ? 0 : b0 * g.nb1 + b1, bB = g.b_shared ? 0 : b0 * g.nb1 + b1;
-  // the tile's A fragments (4 row blocks x NP planes) of one k block are
-  // contiguous, and so are its B fragments; consecutive k blocks are
-  // kstrideA / kstrideB bytes apart
-  const int64_t kstrideA = (int64_t)(g.Mp / RB) * NP * FRAG, kstrideB = (int64_t)(g.Np / RB) * NP * FRAG;
-  const int8_t* gA = g.Aq + bA * g.nkb * kstrideA + (int64_t)(m0 / RB) * NP * FRAG;
-  const int8_t* gB = g.Bq + bB * g.nkb * kstrideB + (int64_t)(n0 / RB) * NP * FRAG;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int wm = (w / WNW) * 32, wn = (w % WNW) * 16 * RJ;
-  const int lr = lane & 15, lk = lane >> 4;
+  OzTile c;
+  c.b0 = bb / (unsigned)g.nb1;
+  c.b1 = bb % (unsigned)g.nb1;
+  c.m0 = (int)mt * TILE;
+  c.n0 = (int)nt * TILE;
+  c.bA = g.a_shared ? 0 : (int64_t)bb;
+  c.bB = g.b_shared ? 0 : (int64_t)bb;
+  return c;
+}
 
-  // wave w copies fragments w, w + 4, .. of the stage: NSL of A, then NSL of B
-  auto copy_stage = [&](int kb, int st) {
-    const int8_t* srcA = gA + (int64_t)kb * kstrideA + 16 * lane;
-    const int8_t* srcB = gB + (int64_t)kb * kstrideB + 16 * lane;
+// One wave's share of a tile.
+template <int NSL>
+struct OzWave {
+  static constexpr int DMAX = NSL, NP = 2 * NSL, STAGE = stage_bytes<NSL>(), STAGE_A = STAGE / 2;
+  const OzGemm& g;
+  int8_t* lds;
+  int w, lane, wm, wn, lr, lk;
+  int64_t kstrideA, kstrideB;
+  v4i rr[2][DMAX + 1], ii[2][DMAX + 1], im[2][DMAX + 1];   // [row block][diagonal]: Ar Br, Ai Bi, Ar Bi + Ai Br
+
+  __device__ OzWave(const OzGemm& gg, int8_t* l, int t) : g(gg), lds(l) {
+    w = __builtin_amdgcn_readfirstlane(t >> 6);
+    lane = t & 63;
+    wm = (w / GEMM_WN) * 32;
+    wn = (w % GEMM_WN) * 16;
+    lr = lane & 15;
+    lk = lane >> 4;
+    // the tile's A fragments (4 row blocks x NP planes) of one k block are
+    // contiguous, and so are its B fragments; consecutive k blocks are
+    // kstrideA / kstrideB bytes apart
+    kstrideA = (int64_t)(g.Mp / RB) * NP * FRAG;
+    kstrideB = (int64_t)(g.Np / RB) * NP * FRAG;
+  }
+  __device__ inline void clear() {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int d = 0; d <= DMAX; ++d) rr[i][d] = ii[i][d] = im[i][d] = v4i{0, 0, 0, 0};
+  }
+  // k block kb of tile c into stage st: wave w copies fragments w, w + 8, .. of A, then of B
+  __device__ inline void copy_stage(const OzTile& c, int kb, int st) const {
+    const int8_t* srcA = g.Aq + (c.bA * g.nkb + kb) * kstrideA + (int64_t)(c.m0 / RB) * NP * FRAG + 16 * lane;
+    const int8_t* srcB = g.Bq + (c.bB * g.nkb + kb) * kstrideB + (int64_t)(c.n0 / RB) * NP * FRAG + 16 * lane;
     int8_t* dst = lds + st * STAGE;
 #pragma unroll
-    for (int it = 0; it < STAGE_A / FRAG / NW; ++it) {
-      const int f = w + NW * it;
+    for (int it = 0; it < STAGE_A / FRAG / GEMM_WAVES; ++it) {
+      const int f = w + GEMM_WAVES * it;
       __builtin_amdgcn_global_load_lds((const void*)(srcA + f * FRAG),
                                        (__attribute__((address_space(3))) void*)(dst + f * FRAG), 16, 0, 0);
     }
 #pragma unroll
-    for (int it = 0; it < STAGE_A / FRAG / NW; ++it) {
-      const int f = w + NW * it;
+    for (int it = 0; it < STAGE_A / FRAG / GEMM_WAVES; ++it) {
+      const int f = w + GEMM_WAVES * it;
       __builtin_amdgcn_global_load_lds((const void*)(srcB + f * FRAG),
                                        (__attribute__((address_space(3))) void*)(dst + STAGE_A + f * FRAG), 16, 0,
                                        0);
     }
-  };
-
-  // exponents of the rows / columns this lane stores (fetched with the first
-  // k block)
-  int ea[2][4], eb[RJ];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int row = m0 + wm + 16 * i + 4 * lk + r;
-      ea[i][r] = row < g.M ? g.EA[bA * g.Mp + row] : INT_MIN;
-    }
-#pragma unroll
-  for (int j = 0; j < RJ; ++j) {
-    const int col = n0 + wn + 16 * j + lr;
-    eb[j] = col < g.N ? g.EB[bB * g.Np + col] : INT_MIN;
   }
-
-  v4i re[2][RJ][DMAX + 1], im[2][RJ][DMAX + 1];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < RJ; ++j)
-#pragma unroll
-      for (int d = 0; d <= DMAX; ++d) { re[i][j][d] = v4i{0, 0, 0, 0}; im[i][j][d] = v4i{0, 0, 0, 0}; }
-
-  copy_stage(0, 0);
-  for (int kb = 0; kb < g.nkb; ++kb) {
-    const int st = kb & 1;
-    // stage st has landed for every wave, and every wave is done with the
-    // stage the next copy overwrites
-    __syncthreads();
-    if (kb + 1 < g.nkb) copy_stage(kb + 1, st ^ 1);
+  // The products of the k block in stage st.  The wave walks its A slices from
+  // the last to the first, so the B fragments it needs grow by one slice per
+  // step and are read from LDS one step ahead of their first use.
+  __device__ inline void compute(int st) {
     const int8_t* sA = lds + st * STAGE + (wm / RB) * NP * FRAG + 16 * lane;
     const int8_t* sB = lds + st * STAGE + STAGE_A + (wn / RB) * NP * FRAG + 16 * lane;
-    // B fragments of slice u: bf[j][2u] (re), bf[j][2u + 1] (im), block column j
-    v4i bf[RJ][NP];
+    v4i br[NSL], bi[NSL];   // B fragments of a slice
 #pragma unroll
-    for (int u = 0; u < NSL && u <= DMAX - (NSL - 1); ++u)
-#pragma unroll
-      for (int j = 0; j < RJ; ++j) {
-        bf[j][2 * u] = lds_frag(sB + (j * NP + 2 * u) * FRAG);
-        bf[j][2 * u + 1] = lds_frag(sB + (j * NP + 2 * u + 1) * FRAG);
-      }
+    for (int u = 0; u < NSL && u <= DMAX - (NSL - 1); ++u) {
+      br[u] = lds_frag(sB + (2 * u) * FRAG);
+      bi[u] = lds_frag(sB + (2 * u + 1) * FRAG);
+    }
     v4i ar = lds_frag(sA + (2 * (NSL - 1)) * FRAG), ai = lds_frag(sA + (2 * (NSL - 1) + 1) * FRAG);
 #pragma unroll
     for (int step = 0; step < 2 * NSL; ++step) {
@@ -545,31 +534,19 @@ __global__ __launch_bounds__(128 * WNW) void oz_gemm_kernel(const OzGemm g) {
       // the slice of B the next step uses first
       if (i == 0 && s >= 1 && DMAX - s + 1 < NSL) {
         const int u = DMAX - s + 1;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          bf[j][2 * u] = lds_frag(sB + (j * NP + 2 * u) * FRAG);
-          bf[j][2 * u + 1] = lds_frag(sB + (j * NP + 2 * u + 1) * FRAG);
-        }
+        br[u] = lds_frag(sB + (2 * u) * FRAG);
+        bi[u] = lds_frag(sB + (2 * u + 1) * FRAG);
       }
-      const v4i nai = neg_bytes(ai);
       // the products with Ar for every slice u of the step, then those with Ai
 #pragma unroll
       for (int u = 0; u < NSL && u + s <= DMAX; ++u) {
-        const int d = s + u;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          re[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, bf[j][2 * u], re[i][j][d], 0, 0, 0);
-          im[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, bf[j][2 * u + 1], im[i][j][d], 0, 0, 0);
-        }
+        rr[i][s + u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, br[u], rr[i][s + u], 0, 0, 0);
+        im[i][s + u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, bi[u], im[i][s + u], 0, 0, 0);
       }
 #pragma unroll
       for (int u = 0; u < NSL && u + s <= DMAX; ++u) {
-        const int d = s + u;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          re[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(nai, bf[j][2 * u + 1], re[i][j][d], 0, 0, 0);
-          im[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ai, bf[j][2 * u], im[i][j][d], 0, 0, 0);
-        }
+        ii[i][s + u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ai, bi[u], ii[i][s + u], 0, 0, 0);
+        im[i][s + u] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ai, br[u], im[i][s + u], 0, 0, 0);
       }
       ar = ar2;
       ai = ai2;
@@ -577,74 +554,70 @@ __global__ __launch_bounds__(128 * WNW) void oz_gemm_kernel(const OzGemm g) {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  // epilogue: lane (lr, lk), register r holds row 4 lk + r, column lr of each 16 x 16 block
+  // exponents of the rows / column this lane stores
+  __device__ inline void load_exps(const OzTile& c, int (&ea)[2][4], int& eb) const {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < RJ; ++j)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int row = m0 + wm + 16 * i + 4 * lk + r, col = n0 + wn + 16 * j + lr;
-        if (row >= g.M || col >= g.N) continue;
-        double vr = (double)re[i][j][DMAX][r], vi = (double)im[i][j][DMAX][r];
-#pragma unroll
-        for (int d = DMAX - 1; d >= 0; --d) {
-          vr = vr * 0.0078125 + (double)re[i][j][d][r];
-          vi = vi * 0.0078125 + (double)im[i][j][d][r];
-        }
-        const int sc = -(sigma_of(ea[i][r]) + sigma_of(eb[j]));
-        oz_store<TO>(g, b0, b1, row, col, ldexp(vr, sc), ldexp(vi, sc));
+        const int row = c.m0 + wm + 16 * i + 4 * lk + r;
+        ea[i][r] = row < g.M ? g.EA[c.bA * g.Mp + row] : INT_MIN;
       }
-}
-
-// Coordinates of logical tile L: within a batch, groups of GM row tiles,
-// column after column (or the batch index fastest when every batch shares A).
-struct OzTile {
-  int m0, n0;
-  int64_t b0, b1, bA, bB;
-};
-__device__ inline OzTile oz_tile(const OzGemm& g, int64_t L, int tiles_m, int tiles_n) {
-  int mt, nt;
-  OzTile c;
-  if (g.batch_major) {
-    const int64_t nb = (int64_t)g.nb0 * g.nb1, bb = L % nb;
-    L /= nb;
-    mt = (int)(L % tiles_m);
-    nt = (int)(L / tiles_m);
-    c.b1 = bb % g.nb1;
-    c.b0 = bb / g.nb1;
-  } else {
-    const int per_batch = tiles_m * tiles_n;
-    const int64_t bb = L / per_batch;
-    const int r = (int)(L - bb * per_batch);
-    const int mg = r / (GM * tiles_n), rem = r - mg * (GM * tiles_n);
-    const int gm = min(GM, tiles_m - mg * GM);   // row tiles in this group
-    nt = rem / gm;
-    mt = mg * GM + (rem - nt * gm);
-    c.b1 = bb % g.nb1;
-    c.b0 = bb / g.nb1;
+    const int col = c.n0 + wn + lr;
+    eb = col < g.N ? g.EB[c.bB * g.Np + col] : INT_MIN;
   }
-  c.m0 = mt * TILE;
-  c.n0 = nt * TILE;
-  c.bA = g.a_shared ? 0 : c.b0 * g.nb1 + c.b1;
-  c.bB = g.b_shared ? 0 : c.b0 * g.nb1 + c.b1;
-  return c;
+  // lane (lr, lk), register r holds row 4 lk + r, column lr of each 16 x 16 block
+  template <class TO>
+  __device__ inline void store(const OzTile& c, const int (&ea)[2][4], int eb) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = c.m0 + wm + 16 * i + 4 * lk + r, col = c.n0 + wn + lr;
+        if (row >= g.M || col >= g.N) continue;
+        double vr = 0.0, vi = 0.0;
+#pragma unroll
+        for (int d = DMAX; d >= 0; --d) {
+          vr = vr * 0.0078125 + (double)(rr[i][d][r] - ii[i][d][r]);
+          vi = vi * 0.0078125 + (double)im[i][d][r];
+        }
+        const int sc = -(sigma_of(ea[i][r]) + sigma_of(eb));
+        oz_store<TO>(g, c.b0, c.b1, row, col, ldexp(vr, sc), ldexp(vi, sc));
+      }
+  }
+};
+
+template <class TO, int NSL>
+__global__ __launch_bounds__(64 * GEMM_WAVES) void oz_gemm_kernel(const OzGemm g) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[2 * stage_bytes<NSL>()];
+  const int tiles_m = (g.M + TILE - 1) / TILE, tiles_n = (g.N + TILE - 1) / TILE;
+  const OzTile c = oz_tile(g, oz_xcd_logical(blockIdx.x, gridDim.x), tiles_m, tiles_n);
+  OzWave<NSL> wv(g, lds, threadIdx.x);
+  int ea[2][4], eb;
+  wv.load_exps(c, ea, eb);   // fetched with the first k block
+  wv.clear();
+  wv.copy_stage(c, 0, 0);
+  for (int kb = 0; kb < g.nkb; ++kb) {
+    // stage kb & 1 has landed for every wave, and every wave is done with the
+    // stage the next copy overwrites
+    __syncthreads();
+    if (kb + 1 < g.nkb) wv.copy_stage(c, kb + 1, (kb & 1) ^ 1);
+    wv.compute(kb & 1);
+  }
+  wv.template store<TO>(c, ea, eb);
 }
 
-// Variant for short k extents (a few k blocks per tile), persistent (waves
-// laid out as in oz_gemm_kernel): each workgroup walks several tiles
-// (workgroup w, on XCD w % 8,
+// Variant for short k extents (a few k blocks per tile), persistent: each
+// workgroup walks several tiles (workgroup w, on XCD w % 8,
 // takes every nx-th tile of that XCD's contiguous range, nx = the XCD's
 // workgroups), so the tiles an XCD runs at once are neighbours in the tile
 // order.  The copy of a tile's first k block is issued with the previous
 // tile's last k block, so the epilogue of one tile runs while the next
 // tile's first stage lands; the exponents of the rows and columns a lane
 // stores are fetched with the tile's last k block.
-template <class TO, int NSL, int WNW>
-__global__ __launch_bounds__(128 * WNW) void oz_gemm_walk_kernel(const OzGemm g, int64_t ntiles) {
-  constexpr int DMAX = NSL, NP = 2 * NSL, STAGE = stage_bytes<NSL>(), STAGE_A = STAGE / 2;
-  constexpr int NW = 2 * WNW, RJ = 4 / WNW;   // waves; column blocks per wave (2 row blocks each)
-  __shared__ __attribute__((aligned(1024))) int8_t lds[2 * STAGE];
+template <class TO, int NSL>
+__global__ __launch_bounds__(64 * GEMM_WAVES) void oz_gemm_walk_kernel(const OzGemm g, int64_t ntiles) {
+  __shared__ __attribute__((aligned(1024))) int8_t lds[2 * stage_bytes<NSL>()];
   const int tiles_m = (g.M + TILE - 1) / TILE, tiles_n = (g.N + TILE - 1) / TILE;
   const int64_t P = gridDim.x, x = blockIdx.x % 8, slot = blockIdx.x / 8;
   const int64_t nx = (P - x + 7) / 8;
@@ -653,156 +626,31 @@ __global__ __launch_bounds__(128 * WNW) void oz_gemm_walk_kernel(const OzGemm g,
   int64_t L = end - per - (x < rem ? 1 : 0) + slot;
   if (L >= end) return;   // uniform over the workgroup
 
-  // the tile's A fragments (4 row blocks x NP planes) of one k block are
-  // contiguous, and so are its B fragments; consecutive k blocks are
-  // kstrideA / kstrideB bytes apart
-  const int64_t kstrideA = (int64_t)(g.Mp / RB) * NP * FRAG, kstrideB = (int64_t)(g.Np / RB) * NP * FRAG;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
-  const int wm = (w / WNW) * 32, wn = (w % WNW) * 16 * RJ;
-  const int lr = lane & 15, lk = lane >> 4;
-
-  // wave w copies fragments w, w + 4, .. of the stage: NSL of A, then NSL of B
-  auto copy_stage = [&](const OzTile& c, int kb, int st) {
-    const int8_t* srcA = g.Aq + c.bA * g.nkb * kstrideA + (int64_t)(c.m0 / RB) * NP * FRAG +
-                         (int64_t)kb * kstrideA + 16 * lane;
-    const int8_t* srcB = g.Bq + c.bB * g.nkb * kstrideB + (int64_t)(c.n0 / RB) * NP * FRAG +
-                         (int64_t)kb * kstrideB + 16 * lane;
-    int8_t* dst = lds + st * STAGE;
-#pragma unroll
-    for (int it = 0; it < STAGE_A / FRAG / NW; ++it) {
-      const int f = w + NW * it;
-      __builtin_amdgcn_global_load_lds((const void*)(srcA + f * FRAG),
-                                       (__attribute__((address_space(3))) void*)(dst + f * FRAG), 16, 0, 0);
-    }
-#pragma unroll
-    for (int it = 0; it < STAGE_A / FRAG / NW; ++it) {
-      const int f = w + NW * it;
-      __builtin_amdgcn_global_load_lds((const void*)(srcB + f * FRAG),
-                                       (__attribute__((address_space(3))) void*)(dst + STAGE_A + f * FRAG), 16, 0,
-                                       0);
-    }
-  };
-  // exponents of the rows / columns this lane stores
-  auto load_exps = [&](const OzTile& c, int (&ea)[2][4], int (&eb)[RJ]) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = c.m0 + wm + 16 * i + 4 * lk + r;
-        ea[i][r] = row < g.M ? g.EA[c.bA * g.Mp + row] : INT_MIN;
-      }
-#pragma unroll
-    for (int j = 0; j < RJ; ++j) {
-      const int col = c.n0 + wn + 16 * j + lr;
-      eb[j] = col < g.N ? g.EB[c.bB * g.Np + col] : INT_MIN;
-    }
-  };
-
+  OzWave<NSL> wv(g, lds, threadIdx.x);
   OzTile cur = oz_tile(g, L, tiles_m, tiles_n);
-  v4i re[2][RJ][DMAX + 1], im[2][RJ][DMAX + 1];
-  // the products of one k block from stage st
-  auto compute = [&](int st) {
-    const int8_t* sA = lds + st * STAGE + (wm / RB) * NP * FRAG + 16 * lane;
-    const int8_t* sB = lds + st * STAGE + STAGE_A + (wn / RB) * NP * FRAG + 16 * lane;
-    // B fragments of slice u: bf[j][2u] (re), bf[j][2u + 1] (im), block column j
-    v4i bf[RJ][NP];
-#pragma unroll
-    for (int u = 0; u < NSL && u <= DMAX - (NSL - 1); ++u)
-#pragma unroll
-      for (int j = 0; j < RJ; ++j) {
-        bf[j][2 * u] = lds_frag(sB + (j * NP + 2 * u) * FRAG);
-        bf[j][2 * u + 1] = lds_frag(sB + (j * NP + 2 * u + 1) * FRAG);
-      }
-    v4i ar = lds_frag(sA + (2 * (NSL - 1)) * FRAG), ai = lds_frag(sA + (2 * (NSL - 1) + 1) * FRAG);
-#pragma unroll
-    for (int step = 0; step < 2 * NSL; ++step) {
-      const int i = step / NSL, s = NSL - 1 - step % NSL;
-      v4i ar2 = ar, ai2 = ai;
-      if (step + 1 < 2 * NSL) {
-        const int i2 = (step + 1) / NSL, s2 = NSL - 1 - (step + 1) % NSL;
-        ar2 = lds_frag(sA + (i2 * NP + 2 * s2) * FRAG);
-        ai2 = lds_frag(sA + (i2 * NP + 2 * s2 + 1) * FRAG);
-      }
-      // the slice of B the next step uses first
-      if (i == 0 && s >= 1 && DMAX - s + 1 < NSL) {
-        const int u = DMAX - s + 1;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          bf[j][2 * u] = lds_frag(sB + (j * NP + 2 * u) * FRAG);
-          bf[j][2 * u + 1] = lds_frag(sB + (j * NP + 2 * u + 1) * FRAG);
-        }
-      }
-      const v4i nai = neg_bytes(ai);
-      // the products with Ar for every slice u of the step, then those with Ai
-#pragma unroll
-      for (int u = 0; u < NSL && u + s <= DMAX; ++u) {
-        const int d = s + u;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          re[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, bf[j][2 * u], re[i][j][d], 0, 0, 0);
-          im[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ar, bf[j][2 * u + 1], im[i][j][d], 0, 0, 0);
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < NSL && u + s <= DMAX; ++u) {
-        const int d = s + u;
-#pragma unroll
-        for (int j = 0; j < RJ; ++j) {
-          re[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(nai, bf[j][2 * u + 1], re[i][j][d], 0, 0, 0);
-          im[i][j][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ai, bf[j][2 * u], im[i][j][d], 0, 0, 0);
-        }
-      }
-      ar = ar2;
-      ai = ai2;
-      // keep each step's MFMAs together, behind the reads issued for the next step
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
   int st = 0;
-  copy_stage(cur, 0, 0);
+  wv.copy_stage(cur, 0, 0);
   for (;;) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < RJ; ++j)
-#pragma unroll
-        for (int d = 0; d <= DMAX; ++d) { re[i][j][d] = v4i{0, 0, 0, 0}; im[i][j][d] = v4i{0, 0, 0, 0}; }
+    wv.clear();
     for (int kb = 0; kb + 1 < g.nkb; ++kb, st ^= 1) {
       // stage st has landed for every wave, and every wave is done with the
       // stage the next copy overwrites
       __syncthreads();
-      copy_stage(cur, kb + 1, st ^ 1);
-      compute(st);
+      wv.copy_stage(cur, kb + 1, st ^ 1);
+      wv.compute(st);
     }
     // the last k block: the exponents the epilogue needs (issued before the
     // next copy, so waiting for them leaves that copy in flight), then the
     // next tile's first k block
     __syncthreads();
-    int ea[2][4], eb[RJ];
-    load_exps(cur, ea, eb);
+    int ea[2][4], eb;
+    wv.load_exps(cur, ea, eb);
     const bool more = L + nx < end;
     const OzTile nxt = oz_tile(g, more ? L + nx : L, tiles_m, tiles_n);
-    if (more) copy_stage(nxt, 0, st ^ 1);
-    compute(st);
+    if (more) wv.copy_stage(nxt, 0, st ^ 1);
+    wv.compute(st);
     st ^= 1;
-    // epilogue: lane (lr, lk), register r holds row 4 lk + r, column lr of each 16 x 16 block
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < RJ; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = cur.m0 + wm + 16 * i + 4 * lk + r, col = cur.n0 + wn + 16 * j + lr;
-          if (row >= g.M || col >= g.N) continue;
-          double vr = (double)re[i][j][DMAX][r], vi = (double)im[i][j][DMAX][r];
-#pragma unroll
-          for (int d = DMAX - 1; d >= 0; --d) {
-            vr = vr * 0.0078125 + (double)re[i][j][d][r];
-            vi = vi * 0.0078125 + (double)im[i][j][d][r];
-          }
-          const int sc = -(sigma_of(ea[i][r]) + sigma_of(eb[j]));
-          oz_store<TO>(g, cur.b0, cur.b1, row, col, ldexp(vr, sc), ldexp(vi, sc));
-        }
+    wv.template store<TO>(cur, ea, eb);
     if (!more) break;
     L += nx;
     cur = nxt;
@@ -901,13 +749,13 @@ void launch_gemm(const OzGemm& g, int64_t tiles, int64_t nkb, bool out_f32, hipS
     // K = 600 and K = 10816 launches walking tiles cost 1-2 %)
     const unsigned grid = (unsigned)std::min<int64_t>(tiles, compute_units());
     // eight waves (two per SIMD): 4-14 % faster than four at the K = nao sites
-    if (out_f32) hipLaunchKernelGGL((oz_gemm_walk_kernel<float2, NSL, 4>), dim3(grid), dim3(512), 0, s, g, tiles);
-    else hipLaunchKernelGGL((oz_gemm_walk_kernel<double2, NSL, 4>), dim3(grid), dim3(512), 0, s, g, tiles);
+    if (out_f32) hipLaunchKernelGGL((oz_gemm_walk_kernel<float2, NSL>), dim3(grid), dim3(64 * GEMM_WAVES), 0, s, g, tiles);
+    else hipLaunchKernelGGL((oz_gemm_walk_kernel<double2, NSL>), dim3(grid), dim3(64 * GEMM_WAVES), 0, s, g, tiles);
   } else if (out_f32) {
     // eight waves (two per SIMD): 1-3 % faster than four on every long-K site
-    hipLaunchKernelGGL((oz_gemm_kernel<float2, NSL, 4>), dim3((unsigned)tiles), dim3(512), 0, s, g);
+    hipLaunchKernelGGL((oz_gemm_kernel<float2, NSL>), dim3((unsigned)tiles), dim3(64 * GEMM_WAVES), 0, s, g);
   } else {
-    hipLaunchKernelGGL((oz_gemm_kernel<double2, NSL, 4>), dim3((unsigned)tiles), dim3(512), 0, s, g);
+    hipLaunchKernelGGL((oz_gemm_kernel<double2, NSL>), dim3((unsigned)tiles), dim3(64 * GEMM_WAVES), 0, s, g);
   }
   GGPU_HIP(hipGetLastError());
 }
