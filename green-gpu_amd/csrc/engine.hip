@@ -5,7 +5,7 @@
 //   Gf        (nk, ns, nts, nao, nao)      G on the full BZ (rotated once per iteration)
 //   Sig_acc   (ink, ns, nts, nao, nao)     Sigma accumulator for the IBZ k
 //   P0        (nts/2, NQ, NQ)              bare bubble of the current q, t < nts/2
-//   P0w/Amat  (nw_b, NQ, NQ)               P0(Omega) -> right-hand side / (1 - P0) factor
+//   P0w/Amat  (q_group, nw_b, NQ, NQ)      P0(Omega) -> right-hand side / (1 - P0) factor of the q solved together
 //   Pt        (nts, NQ, NQ)                dressed polarization of the current q
 //   work      pair-batch intermediates (X1, X2 for P0; Y1, Y2 for Sigma)
 #include "engine.hpp"
@@ -699,8 +699,14 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
   }
   Sig_host_dev.resize((size_t)sym.ink * ns * nts * n2);
   P0.resize((size_t)p0_split * half * Q2);
-  P0w.resize((size_t)nw_b * Q2);
-  Amat.resize((size_t)nw_b * Q2);
+  // The steps of a Dyson solve are short dependent launches with a workgroup or
+  // a few per matrix, and one q has only nw_b (about 40) matrices: several q
+  // are solved together, up to two matrices per CU and 1 GiB of them.  nk = 8,
+  // nao = 26, NQ = 100 (eight q): 4.0 -> 1.5 ms of 14.8 per iteration
+  q_group = (int)std::max<int64_t>(
+      1, std::min<int64_t>({(int64_t)sym.inq, (512 + nw_b - 1) / nw_b, ((int64_t)1 << 30) / (2 * 16 * nw_b * Q2)}));
+  P0w.resize((size_t)q_group * nw_b * Q2);
+  Amat.resize((size_t)q_group * nw_b * Q2);
   Pt.resize((size_t)nts * Q2);
   if (lowp()) Pt32.resize((size_t)nts * Q2);
   if (!sym.q_identity()) {
@@ -709,8 +715,8 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
     Uq_dev.resize(sym.U_q.size());
     GGPU_HIP(hipMemcpy(Uq_dev.get(), sym.U_q.data(), Uq_dev.bytes(), hipMemcpyHostToDevice));
   }
-  info.resize(nw_b);
-  if (solver == GGPU_SOLVER_LU) ipiv.resize((size_t)nw_b * NQ);
+  info.resize((size_t)q_group * nw_b);
+  if (solver == GGPU_SOLVER_LU) ipiv.resize((size_t)q_group * nw_b * NQ);
 
   // pair tables
   const int64_t stride = (int64_t)NQ * n2;
@@ -951,53 +957,58 @@ void GwPlan::p0_for_q(int iq) {
   }
 }
 
-// tau -> Omega, Dyson solve, Omega -> tau for the current q (cugw_qpt.cu:174-358)
-void GwPlan::dyson_for_q() {
+// tau -> Omega of the current P0 into slot `slot` of P0w (cugw_qpt.cu:174-222)
+void GwPlan::to_omega(int slot) {
   const int64_t Q2 = (int64_t)NQ * NQ;
-  const int n = NQ;
-  {
-    GemmDesc g;
-    g.M = nw_b; g.N = (int)Q2; g.K = half - 1; g.KB = p0_split;
-    g.A.ptr = Tf_wt.get(); g.A.rs = half - 1; g.A.cs = 1; g.A.kbs = 0;
-    g.B.ptr = P0.get() + Q2; g.B.rs = Q2; g.B.cs = 1; g.B.kbs = (int64_t)half * Q2;
-    g.C.ptr = P0w.get(); g.C.rs = Q2; g.C.cs = 1;
-    g.alpha_re = 1.0 / sym.nk;
-    g.site = kSiteIR;
-    gemm_on(g, Tf_wt, P0, P0w, stream);
-  }
-  herm_one_minus(P0w.get(), Amat.get(), n, nw_b, stream);
+  GemmDesc g;
+  g.M = nw_b; g.N = (int)Q2; g.K = half - 1; g.KB = p0_split;
+  g.A.ptr = Tf_wt.get(); g.A.rs = half - 1; g.A.cs = 1; g.A.kbs = 0;
+  g.B.ptr = P0.get() + Q2; g.B.rs = Q2; g.B.cs = 1; g.B.kbs = (int64_t)half * Q2;
+  g.C.ptr = P0w.get() + (int64_t)slot * nw_b * Q2; g.C.rs = Q2; g.C.cs = 1;
+  g.alpha_re = 1.0 / sym.nk;
+  g.site = kSiteIR;
+  gemm_on(g, Tf_wt, P0, P0w, stream);
+}
+
+// Dyson solve of the first `slots` slots (cugw_qpt.cu:223-322)
+void GwPlan::solve_dyson(int slots) {
+  const int nmat = slots * nw_b;
+  herm_one_minus(P0w.get(), Amat.get(), NQ, nmat, stream);
   if (solver == GGPU_SOLVER_LU) {
-    lu_solve_dyson();
+    lu_solve_dyson(nmat);
   } else {
-    cholesky_solve_dyson();
+    cholesky_solve_dyson(nmat);
   }
-  {
-    GemmDesc g;
-    g.M = nts; g.N = (int)Q2; g.K = nw_b;
-    g.A.ptr = T_tw.get(); g.A.rs = nw_b; g.A.cs = 1;
-    g.B.ptr = P0w.get(); g.B.rs = Q2; g.B.cs = 1;
-    g.C.ptr = Pt.get(); g.C.rs = Q2; g.C.cs = 1;
-    g.site = kSiteIR;
-    gemm_on(g, T_tw, P0w, Pt, stream);
-  }
+}
+
+// Omega -> tau of slot `slot` (cugw_qpt.cu:323-358)
+void GwPlan::to_tau(int slot) {
+  const int64_t Q2 = (int64_t)NQ * NQ;
+  GemmDesc g;
+  g.M = nts; g.N = (int)Q2; g.K = nw_b;
+  g.A.ptr = T_tw.get(); g.A.rs = nw_b; g.A.cs = 1;
+  g.B.ptr = P0w.get() + (int64_t)slot * nw_b * Q2; g.B.rs = Q2; g.B.cs = 1;
+  g.C.ptr = Pt.get(); g.C.rs = Q2; g.C.cs = 1;
+  g.site = kSiteIR;
+  gemm_on(g, T_tw, P0w, Pt, stream);
   if (lowp()) to_c32(Pt.get(), Pt32.get(), (int64_t)Pt.size(), stream);
 }
 
 // (1 - P0) X = P0 by a batched blocked Cholesky factorisation (potrf /
 // potrs semantics, cugw_qpt.cu:223-264): right-looking, 32-column blocks
 // factored in LDS, trailing updates on the matrix cores; X overwrites P0w.
-void GwPlan::cholesky_solve_dyson() {
+void GwPlan::cholesky_solve_dyson(int nmat) {
   const int64_t Q2 = (int64_t)NQ * NQ;
   const int n = NQ;
   const int nb = 32;
   for (int j0 = 0; j0 < n; j0 += nb) {
     const int jb = std::min(nb, n - j0);
-    chol_diag_block(Amat.get(), n, nw_b, j0, jb, info.get(), stream);
-    chol_panel(Amat.get(), n, nw_b, j0, jb, stream);
+    chol_diag_block(Amat.get(), n, nmat, j0, jb, info.get(), stream);
+    chol_panel(Amat.get(), n, nmat, j0, jb, stream);
     const int rem = n - j0 - jb;
     if (rem > 0) {
       GemmDesc h;
-      h.M = rem; h.N = rem; h.K = jb; h.nb0 = nw_b;
+      h.M = rem; h.N = rem; h.K = jb; h.nb0 = nmat;
       h.A.ptr = Amat.get() + (int64_t)(j0 + jb) * n + j0; h.A.rs = n; h.A.cs = 1; h.A.bs0 = Q2;
       h.B.ptr = Amat.get() + (int64_t)(j0 + jb) * n + j0; h.B.rs = 1; h.B.cs = n; h.B.bs0 = Q2; h.B.conj = 1;
       h.C.ptr = Amat.get() + (int64_t)(j0 + jb) * n + (j0 + jb); h.C.rs = n; h.C.cs = 1; h.C.bs0 = Q2;
@@ -1011,7 +1022,7 @@ void GwPlan::cholesky_solve_dyson() {
     const int ib = std::min(nb, n - i0);
     if (i0 > 0) {
       GemmDesc g;
-      g.M = ib; g.N = n; g.K = i0; g.nb0 = nw_b;
+      g.M = ib; g.N = n; g.K = i0; g.nb0 = nmat;
       g.A.ptr = Amat.get() + (int64_t)i0 * n; g.A.rs = n; g.A.cs = 1; g.A.bs0 = Q2;
       g.B.ptr = P0w.get(); g.B.rs = n; g.B.cs = 1; g.B.bs0 = Q2;
       g.C.ptr = P0w.get() + (int64_t)i0 * n; g.C.rs = n; g.C.cs = 1; g.C.bs0 = Q2;
@@ -1019,7 +1030,7 @@ void GwPlan::cholesky_solve_dyson() {
       g.site = kSiteDyson;
       gemm_on(g, Amat, P0w, P0w, stream);
     }
-    trsm_lower_block(Amat.get(), P0w.get(), n, n, nw_b, i0, ib, stream);
+    trsm_lower_block(Amat.get(), P0w.get(), n, n, nmat, i0, ib, stream);
   }
   const int nblk = (n + nb - 1) / nb;
   for (int bi = nblk - 1; bi >= 0; --bi) {
@@ -1027,7 +1038,7 @@ void GwPlan::cholesky_solve_dyson() {
     const int rest = n - i0 - ib;
     if (rest > 0) {
       GemmDesc g;
-      g.M = ib; g.N = n; g.K = rest; g.nb0 = nw_b;
+      g.M = ib; g.N = n; g.K = rest; g.nb0 = nmat;
       g.A.ptr = Amat.get() + (int64_t)(i0 + ib) * n + i0; g.A.rs = 1; g.A.cs = n; g.A.bs0 = Q2; g.A.conj = 1;
       g.B.ptr = P0w.get() + (int64_t)(i0 + ib) * n; g.B.rs = n; g.B.cs = 1; g.B.bs0 = Q2;
       g.C.ptr = P0w.get() + (int64_t)i0 * n; g.C.rs = n; g.C.cs = 1; g.C.bs0 = Q2;
@@ -1035,7 +1046,7 @@ void GwPlan::cholesky_solve_dyson() {
       g.site = kSiteDyson;
       gemm_on(g, Amat, P0w, P0w, stream);
     }
-    trsm_upper_h_block(Amat.get(), P0w.get(), n, n, nw_b, i0, ib, stream);
+    trsm_upper_h_block(Amat.get(), P0w.get(), n, n, nmat, i0, ib, stream);
   }
 }
 
@@ -1046,19 +1057,19 @@ void GwPlan::cholesky_solve_dyson() {
 // trailing update on the matrix cores; then the pivots are applied to the
 // right-hand side, L (unit lower) and U solved blockwise, and X is
 // Hermitised again (cu_compute_Pq.cu:44-53).  X overwrites P0w.
-void GwPlan::lu_solve_dyson() {
+void GwPlan::lu_solve_dyson(int nmat) {
   const int64_t Q2 = (int64_t)NQ * NQ;
   const int n = NQ;
   const int nb = 32;
   for (int j0 = 0; j0 < n; j0 += nb) {
     const int jb = std::min(nb, n - j0);
-    lu_panel(Amat.get(), n, nw_b, j0, jb, ipiv.get(), info.get(), stream);
-    lu_row_swaps(Amat.get(), n, n, nw_b, ipiv.get(), n, j0, j0 + jb, j0, j0 + jb, stream);
+    lu_panel(Amat.get(), n, nmat, j0, jb, ipiv.get(), info.get(), stream);
+    lu_row_swaps(Amat.get(), n, n, nmat, ipiv.get(), n, j0, j0 + jb, j0, j0 + jb, stream);
     const int rem = n - j0 - jb;
     if (rem > 0) {
-      trsm_unit_lower_cols(Amat.get(), Amat.get(), n, nw_b, j0, jb, j0 + jb, rem, stream);
+      trsm_unit_lower_cols(Amat.get(), Amat.get(), n, nmat, j0, jb, j0 + jb, rem, stream);
       GemmDesc h;   // A22 -= L21 U12
-      h.M = rem; h.N = rem; h.K = jb; h.nb0 = nw_b;
+      h.M = rem; h.N = rem; h.K = jb; h.nb0 = nmat;
       h.A.ptr = Amat.get() + (int64_t)(j0 + jb) * n + j0; h.A.rs = n; h.A.cs = 1; h.A.bs0 = Q2;
       h.B.ptr = Amat.get() + (int64_t)j0 * n + (j0 + jb); h.B.rs = n; h.B.cs = 1; h.B.bs0 = Q2;
       h.C.ptr = Amat.get() + (int64_t)(j0 + jb) * n + (j0 + jb); h.C.rs = n; h.C.cs = 1; h.C.bs0 = Q2;
@@ -1068,12 +1079,12 @@ void GwPlan::lu_solve_dyson() {
     }
   }
   // P X = L U X = B: interchange the rows of B, then L Y = P B, U X = Y
-  lu_row_swaps(P0w.get(), n, n, nw_b, ipiv.get(), n, 0, n, 0, 0, stream);
+  lu_row_swaps(P0w.get(), n, n, nmat, ipiv.get(), n, 0, n, 0, 0, stream);
   for (int i0 = 0; i0 < n; i0 += nb) {
     const int ib = std::min(nb, n - i0);
     if (i0 > 0) {
       GemmDesc g;
-      g.M = ib; g.N = n; g.K = i0; g.nb0 = nw_b;
+      g.M = ib; g.N = n; g.K = i0; g.nb0 = nmat;
       g.A.ptr = Amat.get() + (int64_t)i0 * n; g.A.rs = n; g.A.cs = 1; g.A.bs0 = Q2;
       g.B.ptr = P0w.get(); g.B.rs = n; g.B.cs = 1; g.B.bs0 = Q2;
       g.C.ptr = P0w.get() + (int64_t)i0 * n; g.C.rs = n; g.C.cs = 1; g.C.bs0 = Q2;
@@ -1081,7 +1092,7 @@ void GwPlan::lu_solve_dyson() {
       g.site = kSiteDyson;
       gemm_on(g, Amat, P0w, P0w, stream);
     }
-    trsm_unit_lower_cols(Amat.get(), P0w.get(), n, nw_b, i0, ib, 0, n, stream);
+    trsm_unit_lower_cols(Amat.get(), P0w.get(), n, nmat, i0, ib, 0, n, stream);
   }
   const int nblk = (n + nb - 1) / nb;
   for (int bi = nblk - 1; bi >= 0; --bi) {
@@ -1089,7 +1100,7 @@ void GwPlan::lu_solve_dyson() {
     const int rest = n - i0 - ib;
     if (rest > 0) {
       GemmDesc g;
-      g.M = ib; g.N = n; g.K = rest; g.nb0 = nw_b;
+      g.M = ib; g.N = n; g.K = rest; g.nb0 = nmat;
       g.A.ptr = Amat.get() + (int64_t)i0 * n + (i0 + ib); g.A.rs = n; g.A.cs = 1; g.A.bs0 = Q2;
       g.B.ptr = P0w.get() + (int64_t)(i0 + ib) * n; g.B.rs = n; g.B.cs = 1; g.B.bs0 = Q2;
       g.C.ptr = P0w.get() + (int64_t)i0 * n; g.C.rs = n; g.C.cs = 1; g.C.bs0 = Q2;
@@ -1097,9 +1108,9 @@ void GwPlan::lu_solve_dyson() {
       g.site = kSiteDyson;
       gemm_on(g, Amat, P0w, P0w, stream);
     }
-    trsm_upper_cols(Amat.get(), P0w.get(), n, nw_b, i0, ib, 0, n, stream);
+    trsm_upper_cols(Amat.get(), P0w.get(), n, nmat, i0, ib, 0, n, stream);
   }
-  herm_one_minus(P0w.get(), nullptr, n, nw_b, stream);
+  herm_one_minus(P0w.get(), nullptr, n, nmat, stream);
 }
 
 // Sigma(k, tau) -= sum_{Q,Q'} P~(q, tau)[Q'][Q] V^{Q'}(k,k-q) G(k-q, tau) V^{Q dagger}(k,k-q)
@@ -1190,15 +1201,17 @@ void GwPlan::sigma_for_q(int iq) {
 }
 
 void GwPlan::check_info() {
-  std::vector<int> h(nw_b);
-  GGPU_HIP(hipMemcpy(h.data(), info.get(), nw_b * sizeof(int), hipMemcpyDeviceToHost));
+  std::vector<int> h(info.size());
+  GGPU_HIP(hipMemcpy(h.data(), info.get(), info.bytes(), hipMemcpyDeviceToHost));
   for (int w = 0; w < nw_b; ++w)
-    if (h[w] != 0) {
+    for (int g = 0; g < q_group; ++g) {
+      const int col = h[(size_t)g * nw_b + w];
+      if (col == 0) continue;
       if (solver == GGPU_SOLVER_LU)
         throw Error(kErrSingular, "gw: 1 - P0(Omega) is singular (Omega index " + std::to_string(w) +
-                                      ", zero pivot in column " + std::to_string(h[w]) + ")");
+                                      ", zero pivot in column " + std::to_string(col) + ")");
       throw Error(kErrNotPositiveDefinite, "gw: 1 - P0(Omega) is not positive definite (Omega index " +
-                                               std::to_string(w) + ", column " + std::to_string(h[w]) + ")");
+                                               std::to_string(w) + ", column " + std::to_string(col) + ")");
     }
 }
 
@@ -1300,16 +1313,28 @@ void GwPlan::enqueue_iteration(const z64* G_dev, z64* S_dev, bool timed) {
   stage_G(G_dev);
   if (timed) GGPU_HIP(hipEventRecord(ev[1], stream));
   zero(Sig_acc.get(), Sig_acc.size(), stream);
-  zero_int(info.get(), nw_b, stream);
-  for (int iq = share_rank; iq < sym.inq; iq += share_size) {
-    if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 0], stream));
-    last_q = iq;
-    p0_for_q(iq);
-    if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 1], stream));
-    dyson_for_q();
-    if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 2], stream));
-    sigma_for_q(iq);
-    if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 3], stream));
+  zero_int(info.get(), (int64_t)info.size(), stream);
+  const int nq = q_count(), groups = (nq + q_group - 1) / q_group;
+  for (int grp = 0; grp < groups; ++grp) {
+    // even groups of at most q_group of this share's q
+    const int i0 = (int)((int64_t)nq * grp / groups), i1 = (int)((int64_t)nq * (grp + 1) / groups);
+    for (int i = i0; i < i1; ++i) {
+      const int iq = share_rank + i * share_size;
+      if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 0], stream));
+      last_q = iq;
+      last_slot = i - i0;
+      p0_for_q(iq);
+      if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 1], stream));
+      to_omega(i - i0);
+    }
+    solve_dyson(i1 - i0);
+    for (int i = i0; i < i1; ++i) {
+      const int iq = share_rank + i * share_size;
+      to_tau(i - i0);
+      if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 2], stream));
+      sigma_for_q(iq);
+      if (timed) GGPU_HIP(hipEventRecord(qev[4 * iq + 3], stream));
+    }
   }
   if (timed) GGPU_HIP(hipEventRecord(ev[5], stream));
   if (sig_split > 1) {
@@ -1397,13 +1422,18 @@ void GwPlan::iterate_device(const z64* G_dev, z64* S_dev) {
   (void)store.collect_staging_ms();
   enqueue_iteration(G_dev, S_dev, true);
   GGPU_HIP(hipStreamSynchronize(stream));
+  // the Dyson phase (with both transforms) is what the q loop spends besides
   double t_p0 = 0, t_dy = 0, t_sig = 0;
   for (int iq = share_rank; iq < sym.inq; iq += share_size) {
-    float a = 0, b = 0, c = 0;
+    float a = 0, c = 0;
     GGPU_HIP(hipEventElapsedTime(&a, qev[4 * iq + 0], qev[4 * iq + 1]));
-    GGPU_HIP(hipEventElapsedTime(&b, qev[4 * iq + 1], qev[4 * iq + 2]));
     GGPU_HIP(hipEventElapsedTime(&c, qev[4 * iq + 2], qev[4 * iq + 3]));
-    t_p0 += a; t_dy += b; t_sig += c;
+    t_p0 += a; t_sig += c;
+  }
+  if (q_count() > 0) {
+    float all = 0;
+    GGPU_HIP(hipEventElapsedTime(&all, qev[4 * share_rank], ev[5]));
+    t_dy = std::max(0.0, all - t_p0 - t_sig);
   }
   float tot = 0, g = 0, sg = 0;
   GGPU_HIP(hipEventElapsedTime(&tot, ev[0], ev[6]));
@@ -1523,10 +1553,15 @@ void GwPlan::polarization(const double* G, int iq, int which, double* out) {
   VariantGuard vguard(variants, &ozwork);
   GGPU_HIP(hipMemcpyAsync(G_host_dev.get(), G, G_host_dev.bytes(), hipMemcpyHostToDevice, stream));
   stage_G(G_host_dev.get());
-  zero_int(info.get(), nw_b, stream);
+  zero_int(info.get(), (int64_t)info.size(), stream);
   last_q = iq;
+  last_slot = 0;
   p0_for_q(iq);
-  if (which != 0) dyson_for_q();
+  if (which != 0) {
+    to_omega(0);
+    solve_dyson(1);
+    to_tau(0);
+  }
   GGPU_HIP(hipStreamSynchronize(stream));
   (void)store.collect_staging_ms();
   if (which != 0) check_info();
@@ -1560,7 +1595,7 @@ void GwPlan::last_polarization(int which, int* iq, double* out) {
       }
     return;
   }
-  const z64* src = (which == 1) ? P0w.get() : Pt.get();
+  const z64* src = (which == 1) ? P0w.get() + (int64_t)last_slot * nw_b * Q2 : Pt.get();
   const size_t cnt = (which == 1 ? (size_t)nw_b : (size_t)nts) * Q2;
   GGPU_HIP(hipMemcpy(out, src, cnt * sizeof(z64), hipMemcpyDeviceToHost));
 }

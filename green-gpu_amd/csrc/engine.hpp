@@ -202,8 +202,9 @@ struct GwPlan {
   // NQ = 300); the slices are a K-batch of the tau -> Omega transform.
   int p0_split = 8;
   DeviceBuffer<z64> P0, P0w, Amat, Pt, Prot, Ptmp, Uq_dev;
-  DeviceBuffer<int> info;
-  DeviceBuffer<int> ipiv;                // LU pivots, (nw_b, NQ)
+  int q_group = 1;                       // q whose Dyson equations are solved together
+  DeviceBuffer<int> info;                // (q_group, nw_b)
+  DeviceBuffer<int> ipiv;                // LU pivots, (q_group, nw_b, NQ)
   DeviceBuffer<z64> work;
   DeviceBuffer<char> ozwork;            // slices and scales of the int8-emulated FP64 products
   DeviceBuffer<int64_t> bidx_off;       // b * NQ * nao^2
@@ -240,6 +241,7 @@ struct GwPlan {
   double tune_wall_ms = 0;
   int batch_limit = 0;                  // pair batches per q (and star member); 0: all
   int last_q = -1;                      // IBZ q whose intermediates P0 / P0w / Pt hold
+  int last_slot = 0;                    // its slot of P0w
   // Graph replay: the iteration's launches captured once into a HIP graph
   // (for the G / Sigma addresses, variants and q share of the capture) and
   // replayed by every later iterate; needs the integrals resident in HBM.
@@ -279,9 +281,12 @@ struct GwPlan {
   void capture(const z64* G_dev_hostlayout, z64* Sigma_dev_hostlayout);
   void drop_graph();
   void p0_for_q(int iq);
-  void dyson_for_q();
-  void cholesky_solve_dyson();
-  void lu_solve_dyson();
+  void to_omega(int slot);
+  void solve_dyson(int slots);
+  void to_tau(int slot);
+  void cholesky_solve_dyson(int nmat);
+  void lu_solve_dyson(int nmat);
+  int q_count() const { return sym.inq > share_rank ? (sym.inq - share_rank + share_size - 1) / share_size : 0; }
   void sigma_for_q(int iq);
 };
 
