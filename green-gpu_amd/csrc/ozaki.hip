@@ -607,7 +607,7 @@ __global__ __launch_bounds__(64 * GEMM_WAVES) void oz_gemm_kernel(const OzGemm g
   wv.template store<TO>(c, ea, eb);
 }
 
-// Variant for short k extents (a few k blocks per tile), persistent: each
+// Variant for short k extents (up to seven k blocks per tile), persistent: each
 // workgroup walks several tiles (workgroup w, on XCD w % 8,
 // takes every nx-th tile of that XCD's contiguous range, nx = the XCD's
 // workgroups), so the tiles an XCD runs at once are neighbours in the tile
@@ -742,11 +742,13 @@ void slice_operand(SliceView v, int64_t nb, hipStream_t s) {
 template <int NSL>
 void launch_gemm(const OzGemm& g, int64_t tiles, int64_t nkb, bool out_f32, hipStream_t s) {
   require(tiles < ((int64_t)1 << 31), "int8 emulation: grid too large");
-  if (nkb <= 4) {
+  if (nkb <= 7) {
     // short k extents: one workgroup per CU (the two LDS stages fill it),
     // each walking tiles, so a tile's first copy hides behind the previous
-    // tile's last k block (K = nao = 104 launches: 5-11 % faster; on the
-    // K = 600 and K = 10816 launches walking tiles cost 1-2 %)
+    // tile's last k block.  K = nao = 104 launches are 5-11 % faster, sig_py at NQ =
+    // 300, 350, 448 (5, 6, 7 k blocks) 2.20 -> 2.10, 2.37 -> 2.27, 5.30 -> 5.18 ms with
+    // four slices and 2.68 -> 2.61, 2.97 -> 2.81, 6.52 -> 6.47 with five; K = 600 (10
+    // blocks) loses 1 and 2 %
     const unsigned grid = (unsigned)std::min<int64_t>(tiles, compute_units());
     // eight waves (two per SIMD): 4-14 % faster than four at the K = nao sites
     if (out_f32) hipLaunchKernelGGL((oz_gemm_walk_kernel<float2, NSL>), dim3(grid), dim3(64 * GEMM_WAVES), 0, s, g, tiles);
