@@ -817,10 +817,10 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_bf16x3_frag_kernel(const 
 
 inline int64_t fb_round(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
-// Bytes of split planes one launch over nb0 batches needs (B padded to TN).
-inline size_t fb_bytes(const GemmDesc& d, int nb0, bool a_shared, bool b_shared, int TN) {
+// Bytes of split planes a launch over nb0 x nb1 batches needs (B padded to TN).
+inline size_t fb_bytes(const GemmDesc& d, int nb0, int nb1, bool a_shared, bool b_shared, int TN) {
   const int64_t kpb = (d.K + FB_KB - 1) / FB_KB, nkb = kpb * d.KB;
-  const int64_t nbA = a_shared ? 1 : (int64_t)nb0 * d.nb1, nbB = b_shared ? 1 : (int64_t)nb0 * d.nb1;
+  const int64_t nbA = a_shared ? 1 : (int64_t)nb0 * nb1, nbB = b_shared ? 1 : (int64_t)nb0 * nb1;
   const int64_t per_row_block = nkb * FB_NP * FB_FRAG;
   return (size_t)(nbA * (fb_round(d.M, FB_TILE) / 16) + nbB * (fb_round(d.N, TN) / 16)) * per_row_block;
 }
@@ -828,11 +828,19 @@ inline size_t fb_bytes(const GemmDesc& d, int nb0, bool a_shared, bool b_shared,
 // Whether the pre-split tile can run this launch with the workspace it has
 // (one batch of its planes must fit).
 inline bool fb_fits(const GemmDesc& d, int TN) {
-  const bool a_shared = d.A.bs0 == 0 && d.A.bs1 == 0 && d.A.off1 == nullptr;
-  const bool b_shared = d.B.bs0 == 0 && d.B.bs1 == 0 && d.B.off1 == nullptr;
-  return g_workspace != nullptr && fb_bytes(d, 1, a_shared, b_shared, TN) <= g_workspace_bytes;
+  return g_workspace != nullptr && fb_bytes(d, 1, 1, false, false, TN) <= g_workspace_bytes;
 }
 
+// Part b0 in [b0s, b0s + nb0), b1 in [b1s, b1s + nb1) of an operand's batches.
+template <class Op>
+inline Op batch_part(Op o, int b0s, int b1s, size_t elem) {
+  o.ptr = (char*)o.ptr + ((int64_t)b0s * o.bs0 + (o.off1 ? 0 : (int64_t)b1s * o.bs1)) * (int64_t)elem;
+  if (o.off1) o.off1 += b1s;
+  return o;
+}
+
+// The launch in parts of nb0c x nb1c batches: their planes fit the workspace,
+// and the split kernel's grid (one z per batch) its limit of 65535.
 template <class TO, int WMW, int WNW, int TN = 128>
 void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
   const bool a_shared = d.A.bs0 == 0 && d.A.bs1 == 0 && d.A.off1 == nullptr;
@@ -840,47 +848,53 @@ void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
   const int kpb = (d.K + FB_KB - 1) / FB_KB;
   const int64_t nkb = (int64_t)kpb * d.KB;
   const int Mp = (int)fb_round(d.M, FB_TILE), Np = (int)fb_round(d.N, TN);
-  int nb0c = d.nb0;   // batches per part: their planes fit the workspace
-  while (nb0c > 1 && fb_bytes(d, nb0c, a_shared, b_shared, TN) > g_workspace_bytes) nb0c = (nb0c + 1) / 2;
-  require(fb_bytes(d, nb0c, a_shared, b_shared, TN) <= g_workspace_bytes, "gemm: split-bf16 workspace too small");
-  require(Mp / 16 <= 65535 && Np / 16 <= 65535, "gemm: split-bf16 operand too large");
+  int nb0c = d.nb0, nb1c = d.nb1;
+  auto fits = [&] {
+    return (int64_t)nb0c * nb1c <= 65535 && fb_bytes(d, nb0c, nb1c, a_shared, b_shared, TN) <= g_workspace_bytes;
+  };
+  while (nb0c > 1 && !fits()) nb0c = (nb0c + 1) / 2;
+  while (nb1c > 1 && !fits()) nb1c = (nb1c + 1) / 2;
+  require(fits(), "gemm: split-bf16 workspace too small");
+  require(Mp / 16 <= 65535 && Np / 16 <= 65535 && (nkb + 3) / 4 < ((int64_t)1 << 31),
+          "gemm: split-bf16 operand too large");
   const size_t elem = d.out_f32 ? sizeof(float2) : sizeof(double2);
-  for (int b0s = 0; b0s < d.nb0; b0s += nb0c) {
-    const int nb = std::min(nb0c, d.nb0 - b0s);
-    const int64_t nbA = a_shared ? 1 : (int64_t)nb * d.nb1, nbB = b_shared ? 1 : (int64_t)nb * d.nb1;
-    int8_t* Aq = static_cast<int8_t*>(g_workspace);
-    int8_t* Bq = Aq + (size_t)nbA * (Mp / 16) * nkb * FB_NP * FB_FRAG;
-    for (int op = 0; op < 2; ++op) {
-      const Operand& o = op == 0 ? d.A : d.B;
-      FbView v;
-      v.src = static_cast<const float2*>(o.ptr) + (int64_t)b0s * o.bs0;
-      // A(m, k) = A[m rs + k cs]; B(k, n) = B[k rs + n cs]: rows are m / n
-      v.row_s = op == 0 ? o.rs : o.cs;
-      v.k_s = op == 0 ? o.cs : o.rs;
-      v.kb_s = o.kbs; v.bs0 = o.bs0; v.bs1 = o.bs1; v.off1 = o.off1;
-      v.rows = op == 0 ? d.M : d.N; v.K = d.K; v.KB = d.KB;
-      v.nb1 = (op == 0 ? a_shared : b_shared) ? 1 : d.nb1;
-      v.conj = o.conj; v.Rp = op == 0 ? Mp : Np; v.kpb = kpb;
-      v.out = op == 0 ? Aq : Bq;
-      const int64_t nbat = op == 0 ? nbA : nbB;
-      require(nbat <= 65535 && (nkb + 3) / 4 < ((int64_t)1 << 31), "gemm: split-bf16 operand too large");
-      hipLaunchKernelGGL(fb_split_kernel, dim3((unsigned)((nkb + 3) / 4), (unsigned)(v.Rp / 16), (unsigned)nbat),
-                         dim3(256), 0, stream, v, nkb);
+  for (int b1s = 0; b1s < d.nb1; b1s += nb1c)
+    for (int b0s = 0; b0s < d.nb0; b0s += nb0c) {
+      const int nb0 = std::min(nb0c, d.nb0 - b0s), nb1 = std::min(nb1c, d.nb1 - b1s);
+      const int64_t nbA = a_shared ? 1 : (int64_t)nb0 * nb1, nbB = b_shared ? 1 : (int64_t)nb0 * nb1;
+      int8_t* Aq = static_cast<int8_t*>(g_workspace);
+      int8_t* Bq = Aq + (size_t)nbA * (Mp / 16) * nkb * FB_NP * FB_FRAG;
+      for (int op = 0; op < 2; ++op) {
+        const Operand o = batch_part(op == 0 ? d.A : d.B, b0s, b1s, sizeof(float2));
+        FbView v;
+        v.src = static_cast<const float2*>(o.ptr);
+        // A(m, k) = A[m rs + k cs]; B(k, n) = B[k rs + n cs]: rows are m / n
+        v.row_s = op == 0 ? o.rs : o.cs;
+        v.k_s = op == 0 ? o.cs : o.rs;
+        v.kb_s = o.kbs; v.bs0 = o.bs0; v.bs1 = o.bs1; v.off1 = o.off1;
+        v.rows = op == 0 ? d.M : d.N; v.K = d.K; v.KB = d.KB;
+        v.nb1 = (op == 0 ? a_shared : b_shared) ? 1 : nb1;
+        v.conj = o.conj; v.Rp = op == 0 ? Mp : Np; v.kpb = kpb;
+        v.out = op == 0 ? Aq : Bq;
+        const int64_t nbat = op == 0 ? nbA : nbB;
+        hipLaunchKernelGGL(fb_split_kernel, dim3((unsigned)((nkb + 3) / 4), (unsigned)(v.Rp / 16), (unsigned)nbat),
+                           dim3(256), 0, stream, v, nkb);
+        GGPU_HIP(hipGetLastError());
+      }
+      const OutOperand c = batch_part(d.C, b0s, b1s, elem);
+      FbGemm g;
+      g.Aq = Aq; g.Bq = Bq; g.M = d.M; g.N = d.N; g.Mp = Mp; g.Np = Np; g.nkb = nkb;
+      g.nb0 = nb0; g.nb1 = nb1; g.a_shared = a_shared; g.b_shared = b_shared;
+      g.batch_major = ((int64_t)nb0 * nb1 > 1) && a_shared;
+      g.C = c.ptr;
+      g.c_rs = c.rs; g.c_cs = c.cs; g.c_bs0 = c.bs0; g.c_bs1 = c.bs1; g.c_off1 = c.off1;
+      g.alpha_re = d.alpha_re; g.alpha_im = d.alpha_im; g.beta_re = d.beta_re; g.beta_im = d.beta_im;
+      const int64_t tiles = (int64_t)(Mp / FB_TILE) * (Np / TN) * nb0 * nb1;
+      require(tiles < ((int64_t)1 << 31), "gemm: grid too large");
+      hipLaunchKernelGGL((gemm_bf16x3_frag_kernel<TO, WMW, WNW, TN>), dim3((unsigned)tiles), dim3(64 * WMW * WNW), 0,
+                         stream, g);
       GGPU_HIP(hipGetLastError());
     }
-    FbGemm g;
-    g.Aq = Aq; g.Bq = Bq; g.M = d.M; g.N = d.N; g.Mp = Mp; g.Np = Np; g.nkb = nkb;
-    g.nb0 = nb; g.nb1 = d.nb1; g.a_shared = a_shared; g.b_shared = b_shared;
-    g.batch_major = (nb * (int64_t)d.nb1 > 1) && a_shared;
-    g.C = static_cast<char*>(d.C.ptr) + (int64_t)b0s * d.C.bs0 * (int64_t)elem;
-    g.c_rs = d.C.rs; g.c_cs = d.C.cs; g.c_bs0 = d.C.bs0; g.c_bs1 = d.C.bs1; g.c_off1 = d.C.off1;
-    g.alpha_re = d.alpha_re; g.alpha_im = d.alpha_im; g.beta_re = d.beta_re; g.beta_im = d.beta_im;
-    const int64_t tiles = (int64_t)(Mp / FB_TILE) * (Np / TN) * nb * d.nb1;
-    require(tiles < ((int64_t)1 << 31), "gemm: grid too large");
-    hipLaunchKernelGGL((gemm_bf16x3_frag_kernel<TO, WMW, WNW, TN>), dim3((unsigned)tiles), dim3(64 * WMW * WNW), 0,
-                       stream, g);
-    GGPU_HIP(hipGetLastError());
-  }
 }
 
 template <class TO, int SITE>
