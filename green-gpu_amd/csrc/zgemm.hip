@@ -407,12 +407,16 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(WPE)))
 }
 
 // A-stationary split-bf16 x3 kernel, for K <= 2 XBK, no K-batch and one A
-// shared by every batch (the G.V products of the P0 and Sigma chains multiply
-// one V by every tau).  A workgroup splits its A tile once, keeps its waves'
-// A fragments (four bf16 planes, both k-steps) in registers and walks `bpw`
-// consecutive batches, staging only B per batch (the next B is loaded while
-// the current one is multiplied).  Per output element the products are
-// accumulated in the order of gemm_bf16x3_big_kernel, so the sums are equal.
+// for the batches b0 of every b1 (the G.V products of the P0 and Sigma chains
+// multiply the V of each (pair, spin) entry by every tau).  A workgroup splits
+// its A tile once, keeps its waves' A fragments (four bf16 planes, both k-steps)
+// in registers and walks `bpw` consecutive b0 of one b1, staging only B per batch
+// (the next B is loaded while the current one is multiplied).  Per output element
+// the products are accumulated in the order of gemm_bf16x3_big_kernel, so the
+// sums are equal.  sig_vg and p0_gvh of all entries of one q in ms, this tile and the
+// fastest that splits V for every tau: nao = 33, NQ = 127, 16 entries 0.43 / 0.55 and 0.24
+// / 0.29; nao = 52, NQ = 220, 8 entries 0.72 / 0.89 and 0.36 / 0.48.  At nao = 13 it is the
+// slower one (0.068 / 0.058).
 template <class TO, bool AKC, bool BKC, int SITE>
 __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) void gemm_bf16x3_astat_kernel(
     const GemmDesc d, int bpw) {
@@ -426,15 +430,19 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
   const int tid = threadIdx.x;
   const int tiles_m = (d.M + TM - 1) / TM;
   const int tiles_n = (d.N + TN - 1) / TN;
-  const int64_t nbatch = (int64_t)d.nb0 * d.nb1;
   // m-tile fastest: the workgroups sharing a run of B tiles sit side by side
   int64_t lg = xcd_logical(blockIdx.x, gridDim.x);
   const int mt = (int)(lg % tiles_m);
   lg /= tiles_m;
   const int nt = (int)(lg % tiles_n);
-  const int64_t chunk = lg / tiles_n;
+  lg /= tiles_n;
+  const int chunks = (d.nb0 + bpw - 1) / bpw;
+  const int b_first = (int)(lg % chunks) * bpw;
+  const int64_t b1 = lg / chunks;
   const int m0 = mt * TM, n0 = nt * TN;
-  const float2* A = static_cast<const float2*>(d.A.ptr);
+  const float2* A = static_cast<const float2*>(d.A.ptr) + (d.A.off1 ? d.A.off1[b1] : b1 * d.A.bs1);
+  const float2* B1 = static_cast<const float2*>(d.B.ptr) + (d.B.off1 ? d.B.off1[b1] : b1 * d.B.bs1);
+  TO* C1 = static_cast<TO*>(d.C.ptr) + (d.C.off1 ? d.C.off1[b1] : b1 * d.C.bs1);
 
   constexpr int GPR = KT / 8;   // groups per row
   int arow[GA], ak0[GA], brow[GB], bk0[GB];
@@ -500,12 +508,10 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
     }
   const v4u sign = v4u{0x80008000u, 0x80008000u, 0x80008000u, 0x80008000u};
 
-  const int64_t b_first = chunk * bpw;
-  const int nb = (int)(nbatch - b_first < bpw ? nbatch - b_first : bpw);
+  const int nb = min(d.nb0 - b_first, bpw);
   float2 rb[GB][8];
   auto gload_b = [&](int j) {
-    const int64_t b = b_first + j, b0 = b / d.nb1, b1 = b % d.nb1;
-    const float2* B = static_cast<const float2*>(d.B.ptr) + b0 * d.B.bs0 + (d.B.off1 ? d.B.off1[b1] : b1 * d.B.bs1);
+    const float2* B = B1 + (int64_t)(b_first + j) * d.B.bs0;
 #pragma unroll
     for (int u = 0; u < GB; ++u) {
       const int gn = n0 + brow[u];
@@ -559,8 +565,7 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
 #undef GGPU_X3_STEP
       }
     }
-    const int64_t b = b_first + j, b0 = b / d.nb1, b1 = b % d.nb1;
-    TO* C = static_cast<TO*>(d.C.ptr) + b0 * d.C.bs0 + (d.C.off1 ? d.C.off1[b1] : b1 * d.C.bs1);
+    TO* C = C1 + (int64_t)(b_first + j) * d.C.bs0;
 #pragma unroll
     for (int i = 0; i < WMB; ++i)
 #pragma unroll
@@ -586,11 +591,10 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(2))) v
   }
 }
 
-// Whether the A-stationary kernel applies: one A for every batch, no
+// Whether the A-stationary kernel applies: one A for every batch b0 of a b1, no
 // K-batch, K within its two k-steps, and several batches to walk.
 inline bool astat_fits(const GemmDesc& d) {
-  return d.A.bs0 == 0 && d.A.bs1 == 0 && d.A.off1 == nullptr && d.KB == 1 && d.K <= 2 * XBK &&
-         (int64_t)d.nb0 * d.nb1 >= 2;
+  return d.A.bs0 == 0 && d.KB == 1 && d.K <= 2 * XBK && d.nb0 >= 2;
 }
 
 thread_local GemmProfiler* g_profiler = nullptr;
@@ -666,7 +670,8 @@ struct FbGemm {
   const int8_t* Bq = nullptr;
   int M = 0, N = 0, Mp = 0, Np = 0;
   int64_t nkb = 0;
-  int nb0 = 1, nb1 = 1, a_shared = 0, b_shared = 0, batch_major = 0;
+  int nb0 = 1, nb1 = 1, batch_major = 0;
+  int64_t a_s0 = 0, a_s1 = 0, b_s0 = 0, b_s1 = 0;   // split matrix of batch (b0, b1): b0 s0 + b1 s1
   void* C = nullptr;
   int64_t c_rs = 0, c_cs = 0, c_bs0 = 0, c_bs1 = 0;
   const int64_t* c_off1 = nullptr;
@@ -690,13 +695,13 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_bf16x3_frag_kernel(const 
   int64_t L = xcd_logical(blockIdx.x, gridDim.x);
   int mt, nt;
   int64_t b0, b1;
-  if (g.batch_major) {
-    const int64_t nb = (int64_t)g.nb0 * g.nb1, bb = L % nb;
-    L /= nb;
+  if (g.batch_major) {   // b0 fastest: the workgroups that share an A panel
+    b0 = L % g.nb0;
+    L /= g.nb0;
     mt = (int)(L % tiles_m);
-    nt = (int)(L / tiles_m);
-    b1 = bb % g.nb1;
-    b0 = bb / g.nb1;
+    L /= tiles_m;
+    nt = (int)(L % tiles_n);
+    b1 = L / tiles_n;
   } else {
     mt = (int)(L % tiles_m);
     L /= tiles_m;
@@ -706,7 +711,7 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_bf16x3_frag_kernel(const 
     b0 = L / g.nb1;
   }
   const int m0 = mt * FB_TILE, n0 = nt * TN;
-  const int64_t bA = g.a_shared ? 0 : b0 * g.nb1 + b1, bB = g.b_shared ? 0 : b0 * g.nb1 + b1;
+  const int64_t bA = b0 * g.a_s0 + b1 * g.a_s1, bB = b0 * g.b_s0 + b1 * g.b_s1;
   const int64_t kstrideA = (int64_t)(g.Mp / 16) * FB_NP * FB_FRAG, kstrideB = (int64_t)(g.Np / 16) * FB_NP * FB_FRAG;
   const int8_t* gA = g.Aq + bA * g.nkb * kstrideA + (int64_t)(m0 / 16) * FB_NP * FB_FRAG;
   const int8_t* gB = g.Bq + bB * g.nkb * kstrideB + (int64_t)(n0 / 16) * FB_NP * FB_FRAG;
@@ -817,10 +822,15 @@ __global__ __launch_bounds__(64 * WMW * WNW) void gemm_bf16x3_frag_kernel(const 
 
 inline int64_t fb_round(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
+// Different matrices of an operand along each batch index (1: shared by all).
+inline int fb_distinct0(const Operand& o, int nb0) { return o.bs0 != 0 ? nb0 : 1; }
+inline int fb_distinct1(const Operand& o, int nb1) { return o.off1 || o.bs1 != 0 ? nb1 : 1; }
+
 // Bytes of split planes a launch over nb0 x nb1 batches needs (B padded to TN).
-inline size_t fb_bytes(const GemmDesc& d, int nb0, int nb1, bool a_shared, bool b_shared, int TN) {
+inline size_t fb_bytes(const GemmDesc& d, int nb0, int nb1, int TN) {
   const int64_t kpb = (d.K + FB_KB - 1) / FB_KB, nkb = kpb * d.KB;
-  const int64_t nbA = a_shared ? 1 : (int64_t)nb0 * nb1, nbB = b_shared ? 1 : (int64_t)nb0 * nb1;
+  const int64_t nbA = (int64_t)fb_distinct0(d.A, nb0) * fb_distinct1(d.A, nb1);
+  const int64_t nbB = (int64_t)fb_distinct0(d.B, nb0) * fb_distinct1(d.B, nb1);
   const int64_t per_row_block = nkb * FB_NP * FB_FRAG;
   return (size_t)(nbA * (fb_round(d.M, FB_TILE) / 16) + nbB * (fb_round(d.N, TN) / 16)) * per_row_block;
 }
@@ -828,7 +838,7 @@ inline size_t fb_bytes(const GemmDesc& d, int nb0, int nb1, bool a_shared, bool 
 // Whether the pre-split tile can run this launch with the workspace it has
 // (one batch of its planes must fit).
 inline bool fb_fits(const GemmDesc& d, int TN) {
-  return g_workspace != nullptr && fb_bytes(d, 1, 1, false, false, TN) <= g_workspace_bytes;
+  return g_workspace != nullptr && fb_bytes(d, 1, 1, TN) <= g_workspace_bytes;
 }
 
 // Part b0 in [b0s, b0s + nb0), b1 in [b1s, b1s + nb1) of an operand's batches.
@@ -843,14 +853,12 @@ inline Op batch_part(Op o, int b0s, int b1s, size_t elem) {
 // and the split kernel's grid (one z per batch) its limit of 65535.
 template <class TO, int WMW, int WNW, int TN = 128>
 void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
-  const bool a_shared = d.A.bs0 == 0 && d.A.bs1 == 0 && d.A.off1 == nullptr;
-  const bool b_shared = d.B.bs0 == 0 && d.B.bs1 == 0 && d.B.off1 == nullptr;
   const int kpb = (d.K + FB_KB - 1) / FB_KB;
   const int64_t nkb = (int64_t)kpb * d.KB;
   const int Mp = (int)fb_round(d.M, FB_TILE), Np = (int)fb_round(d.N, TN);
   int nb0c = d.nb0, nb1c = d.nb1;
   auto fits = [&] {
-    return (int64_t)nb0c * nb1c <= 65535 && fb_bytes(d, nb0c, nb1c, a_shared, b_shared, TN) <= g_workspace_bytes;
+    return (int64_t)nb0c * nb1c <= 65535 && fb_bytes(d, nb0c, nb1c, TN) <= g_workspace_bytes;
   };
   while (nb0c > 1 && !fits()) nb0c = (nb0c + 1) / 2;
   while (nb1c > 1 && !fits()) nb1c = (nb1c + 1) / 2;
@@ -861,9 +869,10 @@ void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
   for (int b1s = 0; b1s < d.nb1; b1s += nb1c)
     for (int b0s = 0; b0s < d.nb0; b0s += nb0c) {
       const int nb0 = std::min(nb0c, d.nb0 - b0s), nb1 = std::min(nb1c, d.nb1 - b1s);
-      const int64_t nbA = a_shared ? 1 : (int64_t)nb0 * nb1, nbB = b_shared ? 1 : (int64_t)nb0 * nb1;
+      const int a0 = fb_distinct0(d.A, nb0), a1 = fb_distinct1(d.A, nb1), b0 = fb_distinct0(d.B, nb0),
+                b1 = fb_distinct1(d.B, nb1);
       int8_t* Aq = static_cast<int8_t*>(g_workspace);
-      int8_t* Bq = Aq + (size_t)nbA * (Mp / 16) * nkb * FB_NP * FB_FRAG;
+      int8_t* Bq = Aq + (size_t)a0 * a1 * (Mp / 16) * nkb * FB_NP * FB_FRAG;
       for (int op = 0; op < 2; ++op) {
         const Operand o = batch_part(op == 0 ? d.A : d.B, b0s, b1s, sizeof(float2));
         FbView v;
@@ -873,19 +882,21 @@ void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
         v.k_s = op == 0 ? o.cs : o.rs;
         v.kb_s = o.kbs; v.bs0 = o.bs0; v.bs1 = o.bs1; v.off1 = o.off1;
         v.rows = op == 0 ? d.M : d.N; v.K = d.K; v.KB = d.KB;
-        v.nb1 = (op == 0 ? a_shared : b_shared) ? 1 : nb1;
+        v.nb1 = op == 0 ? a1 : b1;
         v.conj = o.conj; v.Rp = op == 0 ? Mp : Np; v.kpb = kpb;
         v.out = op == 0 ? Aq : Bq;
-        const int64_t nbat = op == 0 ? nbA : nbB;
-        hipLaunchKernelGGL(fb_split_kernel, dim3((unsigned)((nkb + 3) / 4), (unsigned)(v.Rp / 16), (unsigned)nbat),
+        hipLaunchKernelGGL(fb_split_kernel,
+                           dim3((unsigned)((nkb + 3) / 4), (unsigned)(v.Rp / 16), op == 0 ? a0 * a1 : b0 * b1),
                            dim3(256), 0, stream, v, nkb);
         GGPU_HIP(hipGetLastError());
       }
       const OutOperand c = batch_part(d.C, b0s, b1s, elem);
       FbGemm g;
       g.Aq = Aq; g.Bq = Bq; g.M = d.M; g.N = d.N; g.Mp = Mp; g.Np = Np; g.nkb = nkb;
-      g.nb0 = nb0; g.nb1 = nb1; g.a_shared = a_shared; g.b_shared = b_shared;
-      g.batch_major = ((int64_t)nb0 * nb1 > 1) && a_shared;
+      g.nb0 = nb0; g.nb1 = nb1;
+      g.a_s0 = a0 > 1 ? a1 : 0; g.a_s1 = a1 > 1 ? 1 : 0;
+      g.b_s0 = b0 > 1 ? b1 : 0; g.b_s1 = b1 > 1 ? 1 : 0;
+      g.batch_major = nb0 > 1 && a0 == 1;
       g.C = c.ptr;
       g.c_rs = c.rs; g.c_cs = c.cs; g.c_bs0 = c.bs0; g.c_bs1 = c.bs1; g.c_off1 = c.off1;
       g.alpha_re = d.alpha_re; g.alpha_im = d.alpha_im; g.beta_re = d.beta_re; g.beta_im = d.beta_im;
@@ -901,10 +912,9 @@ template <class TO, int SITE>
 void launch_bf16x3_astat(const GemmDesc& d, hipStream_t stream) {
   constexpr int TM = 64, TN = 64;
   const int64_t tiles = (int64_t)((d.M + TM - 1) / TM) * ((d.N + TN - 1) / TN);
-  const int64_t nbatch = (int64_t)d.nb0 * d.nb1;
   // batches per workgroup: as many as keep about 2048 workgroups in the grid
-  const int bpw = (int)std::max<int64_t>(1, std::min<int64_t>(16, tiles * nbatch / 2048));
-  const int64_t total = tiles * ((nbatch + bpw - 1) / bpw);
+  const int bpw = (int)std::max<int64_t>(1, std::min<int64_t>(16, tiles * d.nb0 * d.nb1 / 2048));
+  const int64_t total = tiles * ((d.nb0 + bpw - 1) / bpw) * d.nb1;
   require(total < (int64_t)1 << 31, "gemm: grid too large");
   dim3 grid((unsigned)total), block(NTHREADS);
   const bool akc = (d.A.cs == 1) || (d.A.rs != 1);

@@ -90,8 +90,8 @@ enum {
   kBf16Tile64x64 = 0, kBf16Tile128x64 = 1, kBf16Tile64x128 = 4, kBf16Tile160x64 = 5,
   kBf16Tile96x64W3 = 6, kBf16Tile64x96W3 = 7, kBf16Tile64x64W3 = 8,
   // 64 x 64, A split once and kept in registers while the workgroup walks
-  // several batches (one A for every batch, K <= 64, no K-batch; other
-  // launches take the 64 x 64 three-wave tile)
+  // several batches (one A for the batches b0 of every b1, K <= 64, no K-batch;
+  // other launches take the 64 x 64 three-wave tile)
   kBf16TileAstat64x64 = 9,
   // 128 x 128 from operands split once into fragment-native bf16 planes in
   // the plan's workspace (no workspace: the 160 x 64 tile)
