@@ -1349,6 +1349,17 @@ void GwPlan::enqueue_iteration(const z64* G_dev, z64* S_dev, bool timed) {
   if (timed) GGPU_HIP(hipEventRecord(ev[6], stream));
 }
 
+// What last_polarization reads after a whole iteration: also after a replay,
+// where enqueue_iteration does not run and a polarization call may have come
+// between.
+void GwPlan::note_last_q() {
+  const int nq = q_count();
+  if (nq == 0) return;
+  const int groups = (nq + q_group - 1) / q_group;
+  last_q = share_rank + (nq - 1) * share_size;
+  last_slot = nq - 1 - (int)((int64_t)nq * (groups - 1) / groups);
+}
+
 void GwPlan::drop_graph() {
   if (gexec) (void)hipGraphExecDestroy(gexec);
   gexec = nullptr;
@@ -1405,6 +1416,7 @@ void GwPlan::iterate_device(const z64* G_dev, z64* S_dev) {
     }
     GGPU_HIP(hipEventRecord(ev[0], stream));
     GGPU_HIP(hipGraphLaunch(gexec, stream));
+    note_last_q();
     GGPU_HIP(hipEventRecord(ev[6], stream));
     GGPU_HIP(hipStreamSynchronize(stream));
     float tot = 0;
@@ -1523,6 +1535,7 @@ void GwBatch::run() {
   if (stale) capture();
   GGPU_HIP(hipEventRecord(t0, stream));
   GGPU_HIP(hipGraphLaunch(exec, stream));
+  for (auto* p : plans) p->note_last_q();
   GGPU_HIP(hipEventRecord(t1, stream));
   GGPU_HIP(hipStreamSynchronize(stream));
   float ms = 0;

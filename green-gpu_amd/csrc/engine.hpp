@@ -275,6 +275,7 @@ struct GwPlan {
   // phase events around them.
   void enqueue_iteration(const z64* G_dev_hostlayout, z64* Sigma_dev_hostlayout, bool timed);
   void check_info();
+  void note_last_q();
 
  private:
   void stage_G(const z64* G_dev_hostlayout);
