@@ -217,9 +217,7 @@ int ggpu_gw_set_q_share(ggpu_gw_plan* plan, int rank, int size) {
   return guarded([&] {
     ggpu::require(plan && plan->impl, "NULL plan");
     ggpu::require(size >= 1 && rank >= 0 && rank < size, "q share: need 0 <= rank < size");
-    plan->impl->share_rank = rank;
-    plan->impl->share_size = size;
-    plan->impl->invalidate_graph();
+    plan->impl->set_share(rank, size);
   });
 }
 

@@ -699,14 +699,7 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
   }
   Sig_host_dev.resize((size_t)sym.ink * ns * nts * n2);
   P0.resize((size_t)p0_split * half * Q2);
-  // The steps of a Dyson solve are short dependent launches with a workgroup or
-  // a few per matrix, and one q has only nw_b (about 40) matrices: several q
-  // are solved together, up to two matrices per CU and 1 GiB of them.  nk = 8,
-  // nao = 26, NQ = 100 (eight q): 4.0 -> 1.5 ms of 14.8 per iteration
-  q_group = (int)std::max<int64_t>(
-      1, std::min<int64_t>({(int64_t)sym.inq, (512 + nw_b - 1) / nw_b, ((int64_t)1 << 30) / (2 * 16 * nw_b * Q2)}));
-  P0w.resize((size_t)q_group * nw_b * Q2);
-  Amat.resize((size_t)q_group * nw_b * Q2);
+  size_dyson();
   Pt.resize((size_t)nts * Q2);
   if (lowp()) Pt32.resize((size_t)nts * Q2);
   if (!sym.q_identity()) {
@@ -715,8 +708,6 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
     Uq_dev.resize(sym.U_q.size());
     GGPU_HIP(hipMemcpy(Uq_dev.get(), sym.U_q.data(), Uq_dev.bytes(), hipMemcpyHostToDevice));
   }
-  info.resize((size_t)q_group * nw_b);
-  if (solver == GGPU_SOLVER_LU) ipiv.resize((size_t)q_group * nw_b * NQ);
 
   // pair tables
   const int64_t stride = (int64_t)NQ * n2;
@@ -861,6 +852,43 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
   GGPU_HIP(hipMemcpy(sig_dst.get(), dst.data(), dst.size() * sizeof(int64_t), hipMemcpyHostToDevice));
 
   rot.init(sym, nao, ns, nts, stream);
+}
+
+// The steps of a Dyson solve are short dependent launches with a workgroup or
+// a few per matrix, and one q has only nw_b (about 40) matrices: several q of
+// the share are solved together, up to two matrices per CU and 1 GiB of them.
+// nk = 8, nao = 26, NQ = 100 (eight q): 4.0 -> 1.5 ms of 14.8 per iteration.
+// What last_polarization reads moves along.
+void GwPlan::size_dyson() {
+  const int64_t per = (int64_t)nw_b * NQ * NQ;
+  const int slots = (int)std::max<int64_t>(
+      1, std::min<int64_t>({(int64_t)(sym.inq + share_size - 1) / share_size, (512 + nw_b - 1) / nw_b,
+                            ((int64_t)1 << 30) / (2 * 16 * per)}));
+  if (slots == q_group) return;
+  DeviceBuffer<z64> p((size_t)slots * per), a((size_t)slots * per);
+  DeviceBuffer<int> in((size_t)slots * nw_b), piv(solver == GGPU_SOLVER_LU ? (size_t)slots * nw_b * NQ : 0);
+  if (last_q >= 0) {
+    GGPU_HIP(hipMemcpyAsync(p.get(), P0w.get() + last_slot * per, per * sizeof(z64), hipMemcpyDeviceToDevice, stream));
+    last_slot = 0;
+  }
+  GGPU_HIP(hipStreamSynchronize(stream));
+  P0w = std::move(p);
+  Amat = std::move(a);
+  info = std::move(in);
+  ipiv = std::move(piv);
+  q_group = slots;
+}
+
+void GwPlan::set_share(int rank, int size) {
+  share_rank = rank;
+  share_size = size;
+  invalidate_graph();
+  try {
+    size_dyson();
+  } catch (const Error& e) {
+    if (e.code != kErrMemory) throw;
+    (void)hipGetLastError();   // the buffers of the old share serve too
+  }
 }
 
 GwPlan::~GwPlan() {

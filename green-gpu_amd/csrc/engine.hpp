@@ -202,7 +202,7 @@ struct GwPlan {
   // NQ = 300); the slices are a K-batch of the tau -> Omega transform.
   int p0_split = 8;
   DeviceBuffer<z64> P0, P0w, Amat, Pt, Prot, Ptmp, Uq_dev;
-  int q_group = 1;                       // q whose Dyson equations are solved together
+  int q_group = 0;                       // q whose Dyson equations are solved together
   DeviceBuffer<int> info;                // (q_group, nw_b)
   DeviceBuffer<int> ipiv;                // LU pivots, (q_group, nw_b, NQ)
   DeviceBuffer<z64> work;
@@ -228,6 +228,7 @@ struct GwPlan {
   // This device's share of the IBZ q-points: iq = share_rank, share_rank +
   // share_size, ... (the partial Sigma of all shares sums to the full one).
   int share_rank = 0, share_size = 1;
+  void set_share(int rank, int size);
   bool profiling = false;
   SiteProfiler prof;
   std::vector<hipEvent_t> qev;          // per-q phase events
@@ -281,6 +282,7 @@ struct GwPlan {
   void stage_G(const z64* G_dev_hostlayout);
   void capture(const z64* G_dev_hostlayout, z64* Sigma_dev_hostlayout);
   void drop_graph();
+  void size_dyson();
   void p0_for_q(int iq);
   void to_omega(int slot);
   void solve_dyson(int slots);
