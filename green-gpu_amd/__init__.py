@@ -121,10 +121,13 @@ EXPORTED = ["ggpu_last_error", "ggpu_device_count", "ggpu_device_memory",
             "ggpu_gw_plan_destroy"]
 
 # Launch variants of the contraction GEMMs (ids as the library numbers them):
-# FP64 / FP32 LDS k-depth and waves-per-SIMD register allocation, split-bf16
-# workgroup tiles; in the int8 modes the emulation with the mode's slices
-# ("int8") or with five slices ("int8x5", offered to four-slice plans).
-VARIANTS_MFMA = {8: "bk8", 16: "bk16", 83: "bk8_w3", 84: "bk8_w4", 200: "int8", 201: "int8x5"}
+# workgroup tiles, where "by_shape" is the one that the shape chooses; in the
+# int8 modes the emulation with the mode's slices ("int8") or with five slices
+# ("int8x5", offered to four-slice plans), or the FP64 kernel with the tile that
+# the shape chooses, under the name that reports of these modes have for it.
+VARIANTS_F64 = {8: "64x64", 16: "48x64", 83: "by_shape"}
+VARIANTS_F32 = {8: "64x64", 16: "128x64", 83: "by_shape"}
+VARIANTS_INT8 = {83: "bk8_w3", 200: "int8", 201: "int8x5"}
 VARIANTS_BF16 = {0: "64x64", 1: "128x64", 4: "64x128", 5: "160x64", 6: "96x64_w3", 7: "64x96_w3", 8: "64x64_w3",
                  9: "64x64_astat", 10: "128x128_presplit", 11: "128x128_presplit_w8",
                  12: "128x128_presplit_w16", 13: "128x192_presplit_w8"}
@@ -632,7 +635,7 @@ class GwKernel:
 
     def variant_name(self, v):
         """Readable name of a launch variant id in this plan's precision."""
-        names = VARIANTS_BF16 if self.precision == "bf16x3" else VARIANTS_MFMA
+        names = {"fp64": VARIANTS_F64, "fp32": VARIANTS_F32, "bf16x3": VARIANTS_BF16}.get(self.precision, VARIANTS_INT8)
         return "default" if v == -1 else names.get(v, str(v))
 
     def autotune(self, G, rounds=2, batches=1):

@@ -111,11 +111,10 @@ enum {
 enum { kVariantInt8 = 200, kVariantInt8x5 = 201 };
 // Launch variant per call site for the launches of the calling thread
 // (table of kNumSites entries, -1: the built-in choice; nullptr: none):
-// for FP64 8 or 16 forces the 64 x 64 or 48 x 64 workgroup tile and 83 takes
-// the tile chosen by the shape; for FP32 8 or 16 forces the LDS k-depth, 83
-// k-depth 8 with registers allocated for 3 waves per SIMD (all give the same
-// sums); for split-bf16 a kBf16Tile* value; in the int8 modes kVariantInt8 or an
-// FP64 kernel variant.
+// for FP64 8 or 16 forces the 64 x 64 or 48 x 64 workgroup tile, for FP32 64 x
+// 64 or 128 x 64, and 83 takes the tile chosen by the shape (all give the same
+// sums); for split-bf16 a kBf16Tile* value; in the int8 modes kVariantInt8,
+// kVariantInt8x5 or an FP64 kernel variant.
 void set_site_variants(const int* table);
 // Device workspace of the Compute::I8X5 / I8X4 launches of the calling thread
 // (nullptr: none; such launches then fail with an error).

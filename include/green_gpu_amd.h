@@ -368,8 +368,8 @@ int ggpu_gw_graph_captures(ggpu_gw_plan* plan, int* captures);
  * an iteration): the P0 and Sigma chains of the first q of this plan's share,
  * `batches` pair batches per chain (and per star member), best of `rounds`
  * (1 .. 8).  Candidates (variant ids): for FP64 the workgroup tile chosen by
- * the shape (83), 64 x 64 (8) or 48 x 64 (16); for FP32 the LDS k-depth and
- * waves-per-SIMD register allocation (8, 16, 83); the workgroup tile for
+ * the shape (83), 64 x 64 (8) or 48 x 64 (16); for FP32 the same with 128 x 64
+ * (16); the workgroup tile for
  * split-bf16 (0, 1, 4 .. 9; 10 .. 12: 128 x 128 from operands split once into
  * bf16 planes in the plan's workspace, four, eight or sixteen waves; 13:
  * 128 x 192, eight waves); in the
