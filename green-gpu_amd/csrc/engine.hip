@@ -808,8 +808,12 @@ GwPlan::GwPlan(int nao_, int nso_, int ns_, int NQ_, int nts_, int nw_b_, const 
   if (!lowp()) {
     // with up to two 64 x 32 tiles per CU in a Sigma contraction launch, slices
     // of at least 8 auxiliary functions for about four per CU: nk = 1, nao = 10,
-    // NQ = 154 (two-component) 168 -> 60 us; above that the gain is under 2 %
-    // (the complex64 modes keep one FP32 sum over all Q)
+    // NQ = 154 (two-component) 168 -> 60 us; four (pair, spin) entries at nao = 33
+    // and 41, NQ = 4 nao, nts = 62 one slice -> as many as here 22 -> 38 and 33 -> 34
+    // TFLOP/s.  Above the line eight forced slices gain too (nao = 99 54 -> 72, 104 45
+    // -> 66, 3 - 5 % of an iteration), for eight accumulators and their sum: the
+    // line has not been moved there.  (The complex64 modes keep one FP32 sum over
+    // all Q.)
     const int64_t sig = (int64_t)Sig_host_dev.size();
     const int64_t tiles = (int64_t)((nts * nao + 63) / 64) * ((nao + 31) / 32) * ns * std::min(kb, sym.ink);
     const int64_t split = tiles > 512 ? 1 : std::min<int64_t>({(1024 + tiles - 1) / tiles, NQ / 8, ((int64_t)1 << 26) / sig});

@@ -240,7 +240,10 @@ constexpr TileShape kTileShape[kTiles] = {
 // SIMD to hide latencies, plus the tile's operand traffic (rows + columns).
 // Fitted to 60 shapes of the HF / GW contractions (nao 10 to 104, NQ 64 to
 // 600) timed with every tile: the choice is within 1 % of the fastest tile on
-// (geometric) average.  Against a 64 x 64 tile everywhere it is 1.3 - 2.2x
+// (geometric) average over all sites.  At sig_contract alone (four entries, NQ =
+// 4 nao, nts = 62) it is within 3 % at nao = 64, 75, 80, but takes 64 x 16 at
+// nao = 41, 100 and 104 and then has 34, 37, 45 TFLOP/s where 64 x 48 or 64 x 112
+// have 48, 51, 55.  Against a 64 x 64 tile everywhere it is 1.3 - 2.2x
 // faster where an extent is just above a multiple of 64 (nao = 72: p0_gvh
 // 46 -> 69 TFLOP/s) or the grid is small (nao = 26, NQ = 100: p0_contract
 // 20 -> 33, sig_vg 20 -> 36).
