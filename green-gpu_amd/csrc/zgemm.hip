@@ -860,8 +860,8 @@ void launch_bf16x3_frag(const GemmDesc& d, hipStream_t stream) {
   auto fits = [&] {
     return (int64_t)nb0c * nb1c <= 65535 && fb_bytes(d, nb0c, nb1c, TN) <= g_workspace_bytes;
   };
+  while (nb1c > 1 && !fits()) nb1c = (nb1c + 1) / 2;   // b0 last: what its batches share is split once
   while (nb0c > 1 && !fits()) nb0c = (nb0c + 1) / 2;
-  while (nb1c > 1 && !fits()) nb1c = (nb1c + 1) / 2;
   require(fits(), "gemm: split-bf16 workspace too small");
   require(Mp / 16 <= 65535 && Np / 16 <= 65535 && (nkb + 3) / 4 < ((int64_t)1 << 31),
           "gemm: split-bf16 operand too large");
