@@ -269,7 +269,7 @@ int ggpu_gw_staging_ms(ggpu_gw_plan* plan, double* ms);
  * contribution (still divided by nk), so the Sigma of shares 0 .. size-1
  * sum to the full one.  The reference's per-device q loop,
  * cugw_utils.cu:115 (q_ibz_idx = devices_rank; q_ibz_idx += devices_size).
- * Default: rank 0 of 1. */
+ * The buffers of the Dyson solve are sized by the share.  Default: rank 0 of 1. */
 int ggpu_gw_set_q_share(ggpu_gw_plan* plan, int rank, int size);
 int ggpu_gw_load_integrals(ggpu_gw_plan* plan, const double* V_stored);
 int ggpu_gw_synth_integrals(ggpu_gw_plan* plan, uint64_t seed, double sigma);
